@@ -4,14 +4,12 @@
 // writes run in the QKV GEMM's epilogue, SwiGLU in the gate/up GEMM's, and
 // the residual adds of the K-split O and down GEMMs in the next RMSNorm.
 //
-// GEMM: C[M x N] = A[M x K] . W[N x K]^T with natural FP16 weights on
-// v_mfma_f32_32x32x16_f16. The FP32 activations are split exactly into
-// hi = fp16(a) and lo = fp16(a - hi) (a - hi is exact in FP32), and both
-// halves are multiplied: about 22 significant bits of each activation enter
-// the FP32 accumulation, close to the reference's FP32 SGEMM
-// (engine/core.cpp:293-294) at twice the MFMA work of a plain FP16 GEMM.
-// Each output element's K order is fixed by its column, so a row's result
-// does not depend on how many rows the chunk holds.
+// The GEMMs (prefill_gemm.hpp) multiply FP16 hi + lo planes of the FP32
+// activations by natural FP16 weights: about 22 significant bits of each
+// activation enter the FP32 accumulation, close to the reference's FP32 SGEMM
+// (engine/core.cpp:293-294) at twice the MFMA work of a plain FP16 GEMM. Each
+// output element's K order is fixed by its column, so a row's result does not
+// depend on how many rows the chunk holds.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -21,14 +19,10 @@
 #include "half_split.hpp"
 #include "kernels.hpp"
 #include "prefill.hpp"
+#include "prefill_gemm.hpp"
 
 namespace qwen_hip {
 namespace {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float h2f(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
 __device__ __forceinline__ uint16_t f2h(float f) { return to_half_bits(f); }
@@ -39,490 +33,12 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// C[M x N] (+)= A[M x K] . W[N x K]^T on the matrix cores
-// (v_mfma_f32_32x32x16_f16). A arrives as two FP16 planes written by the
-// kernel that produced it, hi = fp16(a) and lo = fp16(a - hi) (a - hi is
-// exact in FP32), W as its FP16 values; every product runs twice (hi, lo), so
-// products are exact and sums FP32. Workgroup tile BM x 128 (BM = 128, 64 or
-// 32), K in steps of 64 through a ring of LDS stages filled by direct global
-// -> LDS loads (global_load_lds_dwordx4) one or two steps ahead of the matrix
-// cores, one barrier per step. A wave retires roughly one 1 KiB load
-// instruction per 240 cycles on this chip, so the loads are spread over 16
-// (BM = 128) or 8 waves per workgroup; 4 (BM = 64: 8) of them also run the
-// MFMAs, each on 64x64 (BM = 128) or 32x32 tiles of C. Epilogues stage C in LDS and write 16 bytes per
-// lane. Each output element accumulates its K terms in the same order
-// whatever BM and its row position, so results do not depend on M or on how
-// rows are grouped.
-constexpr int kTileN = 128, kTileK = 64;
-
-// BN = 192 or 256 (only with BM = 128): 1.5x or 2x the columns per
-// workgroup, so every A byte streamed feeds more MFMA work; 8 MFMA waves, two
-// per SIMD, on 32x96 (BN = 192) or 64x64 tiles (6 waves of 64x64 put two
-// SIMDs' worth of MFMAs on two of the four), and 2 stages of 56 or 64 KiB
-// (the LDS holds no third). At
-// BN = 192 a stage is 56 loads of 1 KiB, so half of the 16 waves issue 4 and
-// half 3 (with two stages every wait is for all of a wave's loads).
-template <int BM, int BN = kTileN>
-struct GemmShape {
-    static_assert(BN == kTileN || ((BN == 192 || BN == 256) && BM == 128), "wide tiles with 128 rows only");
-    static constexpr int kWaves = BM == 128 ? 16 : 8;            // waves per workgroup (all load)
-    static constexpr int kMma = BM == 64 || BN == 192 || BN == 256 ? 8 : 4;  // waves running the MFMAs
-    static constexpr int TI = BM == 128 && BN != 192 ? 2 : 1;    // 32-row tiles per MFMA wave
-    static constexpr int WR = BM / 32 / TI, WC = kMma / WR;      // MFMA wave grid
-    static constexpr int TJ = BN / WC / 32;                      // 32-column tiles per MFMA wave
-    static constexpr int kASlots = BM * 8, kBSlots = BN * 8;     // 16-byte slots per stage
-    static constexpr int kStageBytes = (2 * kASlots + kBSlots) * 16;
-    static constexpr int kStageLoads = (2 * kASlots + kBSlots) / 64;         // 1 KiB loads per stage
-    static constexpr int kLoads = (kStageLoads + kWaves - 1) / kWaves;       // per thread per stage (at most)
-    static constexpr int kStages = BN == kTileN ? (BM == 128 ? 3 : 4) : 2;
-    static_assert(kStageLoads * 64 == 2 * kASlots + kBSlots && WR * WC == kMma && TJ * WC * 32 == BN,
-                  "tile shape");
-    static_assert(kLoads * kWaves == kStageLoads || kStages == 2, "uneven loads need whole-stage waits");
-};
-
-// LDS operand tiles hold rows of 64 halves (eight 16-byte pieces): piece p of
-// row r sits in 16-byte slot 8 r + (p ^ swz(r)), so the 8 (or 16) lanes
-// served in one LDS cycle read distinct banks.
-__device__ __forceinline__ int swz(int r) { return ((r >> 1) ^ ((r & 1) << 2)) & 7; }
-
-// Work fused into the epilogue. QKV (EPI 4): QK-norm, RoPE and the K/V cache
-// writes of engine/core.cpp:395-406. Gate/up (EPI 3): SwiGLU, written as the
-// FP16 hi / lo planes the down GEMM reads.
-//
-// Range guard of the FP16 split (split_exponent): A row m that its producer
-// split as a * 2^-row_exp[m] has its products scaled back by 2^row_exp[m]
-// (EPI 0, 1, 3, 4; row_exp null: no row was scaled). The SwiGLU epilogue
-// splits each group of 8 activations with its own exponent, stored in
-// act_exp [M][N / 16], and raises act_flag [M][4] (one word per K range of
-// the down GEMM, cleared by the kernel before the gate/up GEMM) to the
-// largest exponent in the range. The down GEMM (EPI 2 with act_flag) runs
-// its plain K loop, and a workgroup whose rows saw a nonzero flag runs the
-// loop again with every group rescaled in LDS to its row's flag exponent
-// and the products scaled back: a row that fits keeps its bits.
-struct GemmEpilogue {
-    const float* q_norm;
-    const float* k_norm;
-    const float* cosines;
-    const float* sines;
-    uint16_t* keys;
-    uint16_t* values;
-    int pos0;
-    int context;
-    uint16_t* act_hi;
-    uint16_t* act_lo;
-    const int* row_exp;
-    int* act_flag;
-    uint8_t* act_exp;
-};
-
-// Exponent of row m in row_exp (0 without one).
-__device__ __forceinline__ float row_scale(const int* row_exp, int m) {
-    return row_exp ? pow2(row_exp[m]) : 1.f;
-}
-
 // FP32 value -> the FP16 hi / lo pair the GEMMs read (hi = fp16(v), lo = fp16(v - hi)).
 __device__ __forceinline__ void split_store(float v, uint16_t* hi, uint16_t* lo, size_t i) {
     _Float16 h, l;
     split_half(v, h, l);
     hi[i] = __builtin_bit_cast(uint16_t, h);
     lo[i] = __builtin_bit_cast(uint16_t, l);
-}
-
-// 16 bytes per lane from global memory straight into LDS at
-// lds + 16 lane (lds wave-uniform); counted by vmcnt like any load.
-__device__ __forceinline__ void load_lds16(const void* src, unsigned char* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
-#endif
-}
-
-// vmcnt <= n (expcnt and lgkmcnt unconstrained).
-template <int n>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(n >= 0 && n < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-// lgkmcnt == 0 (this wave's LDS accesses have completed).
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
-
-// Workgroup barrier without a memory fence: the waits before it already
-// cover the direct-to-LDS loads (a fenced barrier would wait for every load
-// in flight, including the later stages). The empty asm statements keep the
-// compiler from moving LDS accesses across it.
-__device__ __forceinline__ void stage_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// Epilogue: 0 store, 1 add into C (residual), 2 store the partial product
-// of K range blockIdx.z (K / gridDim.z columns) at C + blockIdx.z M N,
-// 3 SwiGLU (W = gate rows then up rows, N = 2F: tile t multiplies gate rows
-// 64t.. and up rows F + 64t.. and stores act[m][64t + i] as FP16 hi / lo),
-// 4 QKV rows (tile t = head t): q heads QK-normed, rotated and stored in the
-// key's chain-permuted order, k heads QK-normed, rotated and written to the
-// cache as FP16, v heads written to the cache.
-template <int BM, int EPI, int BN = kTileN>
-__global__ __launch_bounds__((GemmShape<BM, BN>::kWaves * 64)) void gemm_kernel(
-    const uint16_t* __restrict__ Ah, const uint16_t* __restrict__ Al, const uint16_t* __restrict__ W,
-    float* __restrict__ C, int M, int N, int K, GemmEpilogue ep) {
-    using S = GemmShape<BM, BN>;
-    static_assert(EPI != 4 || BN == kTileN, "the QKV epilogue takes one head per tile");
-    constexpr int kStages = S::kStages, kLoads = S::kLoads, kStageBytes = S::kStageBytes;
-    constexpr int kASlots = S::kASlots, WR = S::WR, TI = S::TI, TJ = S::TJ;
-    // Overlapped operand reads (below) for 2 x 2 MFMA tiles per wave; the
-    // K-split 192-column instance keeps the plain order (8 more registers
-    // would spill there).
-    constexpr bool kPipelined = TI == 2 && TJ == 2 && !(EPI == 2 && BN == 192);
-    constexpr int kThreads = S::kWaves * 64;
-    constexpr int kCPitch = BN + 4;  // floats per row of the staged C tile
-    constexpr int kEpiBytes = BM * kCPitch * 4 + (EPI == 4 ? BM * kHeadDim * 2 : 0);
-    constexpr int kSmem = kStages * kStageBytes > kEpiBytes ? kStages * kStageBytes : kEpiBytes;
-    __shared__ __align__(16) unsigned char smem[kSmem];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // Tile of this workgroup: workgroup w runs on XCD w % 8 (round-robin
-    // dispatch). With 4 or more row tiles per XCD, XCD x takes row tiles
-    // x, x + 8, ... and walks the column tiles (its 32 CUs hold 4 row tiles
-    // x 8 column tiles at a time). With fewer (prompts up to 3 x 8 x BM
-    // rows), f = 4 or 2 XCDs pool their row tiles and split the column tiles
-    // by residue mod f, so that the tiles an XCD runs at once still share
-    // A and W rows in its L2: at 1024 rows 4 x 8 tiles per XCD instead of
-    // 1 x 32 (each W tile fetched by 2 XCDs instead of 8). The grid is
-    // rounded up to whole XCD rows; the extra workgroups have no tile.
-    const int mtiles = (M + BM - 1) / BM, per = (mtiles + 7) / 8, ntiles = N / BN;
-    const int f = per >= 4 ? 1 : per == 1 && ntiles % 4 == 0 ? 4 : ntiles % 2 == 0 ? 2 : 1;
-    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, rows = f * per;
-    const int rr = slot % rows, cc = slot / rows;
-    const int mt = (xcd / f) * f + rr % f + 8 * (rr / f), nt = xcd % f + f * cc;
-    if (mt >= mtiles) return;
-    const int m0 = mt * BM, n0 = nt * BN;
-    const bool mma = wave < S::kMma;
-    const int wm = wave % WR, wn = wave / WR;
-    const int ks = K / gridDim.z, kz = blockIdx.z * ks, nk = ks / kTileK;  // this workgroup's K range
-
-    // Load j of this thread fills slot 64 (wave + kWaves j) + lane of a
-    // stage: a wave-uniform operand plane (A hi, A lo, W) and one 16-byte
-    // piece of a row. A rows past M repeat row M - 1 and are never stored.
-    const uint16_t* src[kLoads];
-#pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-        const int q = 64 * (wave + S::kWaves * j) + lane;
-        if (q < 2 * kASlots) {
-            const int qa = q < kASlots ? q : q - kASlots, r = qa >> 3, p = (qa & 7) ^ swz(r);
-            src[j] = (q < kASlots ? Ah : Al) + size_t(min(m0 + r, M - 1)) * K + kz + 8 * p;
-        } else {
-            const int qb = q - 2 * kASlots, r = qb >> 3, p = (qb & 7) ^ swz(r);
-            const int wr = EPI == 3 ? (r < BN / 2 ? n0 / 2 + r : N / 2 + n0 / 2 + r - BN / 2) : n0 + r;
-            src[j] = W + size_t(wr) * K + kz + 8 * p;
-        }
-    }
-    auto issue = [&](int kt) {
-        unsigned char* stage = smem + (kt % kStages) * kStageBytes;
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j)
-            if (kLoads * S::kWaves == S::kStageLoads || wave + S::kWaves * j < S::kStageLoads)
-                load_lds16(src[j] + kt * kTileK, stage + 1024 * (wave + S::kWaves * j));
-    };
-
-    // Range guard of the down GEMM (EPI 2 with act_flag): the flags of this
-    // workgroup's rows in its K range (lane l: rows m0 + l and m0 + 64 + l),
-    // loaded before the stream so that they have arrived when the loop ends.
-    int flag0 = 0, flag1 = 0;
-    if constexpr (EPI == 2) {
-        if (ep.act_flag != nullptr && lane < BM) {
-            flag0 = ep.act_flag[size_t(min(m0 + lane, M - 1)) * 4 + blockIdx.z];
-            if (BM > 64) flag1 = ep.act_flag[size_t(min(m0 + 64 + lane, M - 1)) * 4 + blockIdx.z];
-        }
-    }
-
-    floatx16 acc[TI][TJ];
-    const int fr = lane & 31;
-    // Rescales the A groups of stage kt in LDS to their row's flag
-    // exponent (the second pass of a guarded down GEMM): exact, being
-    // multiplications of FP16 values by powers of two no greater than 1.
-    auto rescale_stage = [&](int kt) {
-        unsigned char* stage = smem + (kt % kStages) * kStageBytes;
-        for (int q = tid; q < kASlots; q += kThreads) {
-            const int r = q >> 3, p = (q & 7) ^ swz(r), m = min(m0 + r, M - 1);
-            const int er = ep.act_flag[size_t(m) * 4 + blockIdx.z];
-            if (er != 0) {
-                const int e8 = ep.act_exp[size_t(m) * (K / 8) + (kz + kt * kTileK) / 8 + p];
-                const float sc = pow2(e8 - er);
-                half8* h = reinterpret_cast<half8*>(stage + 16 * q);
-                half8* l = reinterpret_cast<half8*>(stage + 16 * (kASlots + q));
-                half8 hv = *h, lv = *l;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    hv[e] = static_cast<_Float16>(static_cast<float>(hv[e]) * sc);
-                    lv[e] = static_cast<_Float16>(static_cast<float>(lv[e]) * sc);
-                }
-                *h = hv;
-                *l = lv;
-            }
-        }
-    };
-    auto k_loop = [&](auto rescale_tag) {
-        constexpr bool kRescale = decltype(rescale_tag)::value;
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int jt = 0; jt < TJ; ++jt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][jt][r] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kStages - 1; ++s)
-            if (s < nk) issue(s);
-        for (int kt = 0; kt < nk; ++kt) {
-            // Step kt has landed once no more than the later steps' loads are
-            // pending; the barrier then also tells every wave that all waves are
-            // done reading the stage the next issue overwrites.
-            if (kt + kStages - 2 < nk)
-                wait_vmcnt<(kStages - 2) * kLoads>();
-            else
-                wait_vmcnt<0>();
-            stage_barrier();
-            if (kt + kStages - 1 < nk) issue(kt + kStages - 1);
-            if constexpr (kRescale) {
-                rescale_stage(kt);
-                wait_lgkm0();
-                stage_barrier();
-            }
-            if (mma) {
-                if constexpr (kPipelined) {
-                    // Operand reads of sub-step sub + 1 overlap the MFMAs of sub:
-                    // the B pair and row tile 0 of sub + 1 are read while row tile
-                    // 1 of sub multiplies, row tile 1 of sub + 1 while row tile 0
-                    // of sub + 1 does. Each accumulator still takes hi then lo of
-                    // sub 0, 1, 2, 3 in turn.
-                    const unsigned char* stage = smem + (kt % kStages) * kStageBytes;
-                    auto read_a = [&](int sub, int i, half8& h, half8& l) {
-                        const int p = 2 * sub + (lane >> 5);
-                        const int ra = (wm * TI + i) * 32 + fr, sa = 8 * ra + (p ^ swz(ra));
-                        h = *reinterpret_cast<const half8*>(stage + 16 * sa);
-                        l = *reinterpret_cast<const half8*>(stage + 16 * (kASlots + sa));
-                    };
-                    auto read_b = [&](int sub, half8 (&b)[TJ]) {
-                        const int p = 2 * sub + (lane >> 5);
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt) {
-                            const int rb = wn * (BN / S::WC) + 32 * jt + fr;
-                            b[jt] = *reinterpret_cast<const half8*>(stage + 16 * (2 * kASlots + 8 * rb + (p ^ swz(rb))));
-                        }
-                    };
-                    half8 a0h, a0l, a1h, a1l, bb[2][TJ];
-                    read_a(0, 0, a0h, a0l);
-                    read_b(0, bb[0]);
-                    read_a(0, 1, a1h, a1l);
-#pragma unroll
-                    for (int sub = 0; sub < 4; ++sub) {
-                        half8(&cur)[TJ] = bb[sub & 1];
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt)
-                            acc[0][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0h, cur[jt], acc[0][jt], 0, 0, 0);
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt)
-                            acc[0][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0l, cur[jt], acc[0][jt], 0, 0, 0);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (sub < 3) {
-                            read_b(sub + 1, bb[(sub + 1) & 1]);
-                            read_a(sub + 1, 0, a0h, a0l);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt)
-                            acc[1][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1h, cur[jt], acc[1][jt], 0, 0, 0);
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt)
-                            acc[1][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1l, cur[jt], acc[1][jt], 0, 0, 0);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if (sub < 3) read_a(sub + 1, 1, a1h, a1l);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                } else {
-                    const unsigned char* stage = smem + (kt % kStages) * kStageBytes;
-#pragma unroll
-                    for (int sub = 0; sub < 4; ++sub) {
-                        const int p = 2 * sub + (lane >> 5);  // k = 16 sub + 8 (lane / 32) .. + 7 of the step
-                        half8 ah[TI], al[TI], bb[TJ];
-#pragma unroll
-                        for (int i = 0; i < TI; ++i) {
-                            const int ra = (wm * TI + i) * 32 + fr, sa = 8 * ra + (p ^ swz(ra));
-                            ah[i] = *reinterpret_cast<const half8*>(stage + 16 * sa);
-                            al[i] = *reinterpret_cast<const half8*>(stage + 16 * (kASlots + sa));
-                        }
-#pragma unroll
-                        for (int jt = 0; jt < TJ; ++jt) {
-                            const int rb = wn * (BN / S::WC) + 32 * jt + fr;
-                            bb[jt] = *reinterpret_cast<const half8*>(stage + 16 * (2 * kASlots + 8 * rb + (p ^ swz(rb))));
-                        }
-#pragma unroll
-                        for (int i = 0; i < TI; ++i)
-#pragma unroll
-                            for (int jt = 0; jt < TJ; ++jt) {
-                                acc[i][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bb[jt], acc[i][jt], 0, 0, 0);
-                                acc[i][jt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bb[jt], acc[i][jt], 0, 0, 0);
-                            }
-                    }
-                }
-            }
-        }
-    };
-    k_loop(std::false_type{});
-    // Every wave read the same flags, so every wave takes the same branch.
-    bool rescaled = false;
-    if constexpr (EPI == 2) {
-        if (ep.act_flag != nullptr && __builtin_amdgcn_ballot_w64(flag0 != 0 || flag1 != 0) != 0) {
-            rescaled = true;
-            stage_barrier();  // every wave is done with the stages (all loads were waited for)
-            k_loop(std::true_type{});
-        }
-    }
-
-    // Stage C in LDS. D layout: lane -> column (lane & 31); register r ->
-    // row 8(r/4) + 4(lane/32) + r%4 of the wave's 32-row tile.
-    float(*ct)[kCPitch] = reinterpret_cast<float(*)[kCPitch]>(smem);
-    stage_barrier();  // every wave is done with the operand stages (all loads were waited for)
-    if (mma) {
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int jt = 0; jt < TJ; ++jt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    ct[(wm * TI + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)]
-                      [wn * (BN / S::WC) + 32 * jt + fr] = acc[i][jt][r];
-    }
-    __syncthreads();
-    if constexpr (EPI <= 2) {
-        // 16-byte pieces: row q / (BN / 4), columns 4 (q % (BN / 4)) .. + 3.
-#pragma unroll
-        for (int q = tid; q < BM * (BN / 4); q += kThreads) {
-            const int row = q / (BN / 4), c4 = q % (BN / 4), m = m0 + row;
-            if (m < M) {
-                float4* c = reinterpret_cast<float4*>(C + (size_t(blockIdx.z) * M + m) * N + n0) + c4;
-                float4 v = *reinterpret_cast<const float4*>(&ct[row][4 * c4]);
-                float sc = 1.f;
-                if constexpr (EPI == 2) {
-                    if (rescaled) sc = pow2(ep.act_flag[size_t(m) * 4 + blockIdx.z]);
-                } else {
-                    sc = row_scale(ep.row_exp, m);
-                }
-                v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
-                if constexpr (EPI == 1) {
-                    const float4 o = *c;
-                    *c = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
-                } else {
-                    *c = v;
-                }
-            }
-        }
-    } else if constexpr (EPI == 3) {
-        // SwiGLU (engine/core.cpp:636-639): task q = row q / (BN / 16), act
-        // columns n0 / 2 + 8 (q % (BN / 16)) .. + 7, stored as one 16-byte
-        // piece per plane (gate in tile columns 0 .. BN / 2 - 1, up after).
-#pragma unroll
-        for (int q = tid; q < BM * (BN / 16); q += kThreads) {
-            const int row = q / (BN / 16), c8 = 8 * (q % (BN / 16)), m = m0 + row;
-            if (m < M) {
-                const float sc = row_scale(ep.row_exp, m);
-                float o[8], big = 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float gate = ct[row][c8 + e] * sc, up = ct[row][BN / 2 + c8 + e] * sc;
-                    const float half_gate = gate * 0.5f;
-                    const float t = tanhf(half_gate);
-                    o[e] = gate * (0.5f + 0.5f * t) * up;
-                    big = fmaxf(big, fabsf(o[e]));
-                }
-                // This group's exponent; the K range's flag holds the largest.
-                const int e8 = split_exponent(big), col = n0 / 2 + c8;
-                const float down = pow2(-e8);
-                half8 hi, lo;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    _Float16 h, l;
-                    split_half(o[e] * down, h, l);
-                    hi[e] = h;
-                    lo[e] = l;
-                }
-                const size_t at = size_t(m) * (N / 2) + col;
-                *reinterpret_cast<half8*>(ep.act_hi + at) = hi;
-                *reinterpret_cast<half8*>(ep.act_lo + at) = lo;
-                ep.act_exp[size_t(m) * (N / 16) + col / 8] = static_cast<uint8_t>(e8);
-                if (e8 != 0) atomicMax(ep.act_flag + size_t(m) * 4 + col / (N / 8), e8);
-            }
-        }
-    } else {
-        // Per row (one wave per row, rows wave, wave + kWaves, ...; lane l on
-        // channels l and l + 64): QK-norm and RoPE in place, the row left in
-        // LDS in its stored order (q: FP32 chain-permuted; k: FP16
-        // chain-permuted; v: FP16), then written out 16 bytes per lane.
-        uint16_t(*ht)[kHeadDim] = reinterpret_cast<uint16_t(*)[kHeadDim]>(smem + BM * kCPitch * 4);
-        const int head = nt, j = lane;
-        const bool is_q = head < kQHeads, is_v = head >= kQHeads + kKVHeads;
-        constexpr int kRows = BM / S::kWaves;
-        if (is_v) {
-#pragma unroll
-            for (int k = 0; k < kRows; ++k) {
-                const int rr = wave + S::kWaves * k;
-                const float sc = row_scale(ep.row_exp, min(m0 + rr, M - 1));
-                ht[rr][j] = f2h(ct[rr][j] * sc);
-                ht[rr][j + 64] = f2h(ct[rr][j + 64] * sc);
-            }
-        } else {
-            const float* w = is_q ? ep.q_norm : ep.k_norm;
-            const float w0 = w[j], w1 = w[j + 64];
-            float rc[kRows], rs[kRows];
-#pragma unroll
-            for (int k = 0; k < kRows; ++k) {
-                const int pos = ep.pos0 + min(m0 + wave + S::kWaves * k, M - 1);
-                rc[k] = ep.cosines[size_t(pos) * 64 + j];
-                rs[k] = ep.sines[size_t(pos) * 64 + j];
-            }
-#pragma unroll
-            for (int k = 0; k < kRows; ++k) {
-                const int rr = wave + S::kWaves * k;
-                const float sc = row_scale(ep.row_exp, min(m0 + rr, M - 1));
-                const float x0 = ct[rr][j] * sc, x1 = ct[rr][j + 64] * sc;
-                const float s0 = x0 * x0, s1 = x1 * x1;
-                double part = static_cast<double>(s0) + static_cast<double>(s1);
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off);
-                const float inv = 1.0f / __builtin_sqrtf(static_cast<float>(part) / 128.0f + 1e-6f);
-                const float n0v = (x0 * inv) * w0, n1v = (x1 * inv) * w1;
-                const float o0 = n0v * rc[k] - n1v * rs[k];
-                const float o1 = n1v * rc[k] + n0v * rs[k];
-                if (is_q) {
-                    ct[rr][kperm(j)] = o0;  // the row's reads above came first
-                    ct[rr][kperm(j + 64)] = o1;
-                } else {
-                    ht[rr][kperm(j)] = f2h(o0);
-                    ht[rr][kperm(j + 64)] = f2h(o1);
-                }
-            }
-        }
-        __syncthreads();
-        if (is_q) {
-#pragma unroll
-            for (int q = tid; q < BM * 32; q += kThreads) {
-                const int row = q >> 5, c4 = q & 31, m = m0 + row;
-                if (m < M)
-                    reinterpret_cast<float4*>(C + size_t(m) * N + head * kHeadDim)[c4] =
-                        *reinterpret_cast<const float4*>(&ct[row][4 * c4]);
-            }
-        } else {
-            uint16_t* cache = (is_v ? ep.values + size_t(head - kQHeads - kKVHeads) * ep.context * kHeadDim
-                                    : ep.keys + size_t(head - kQHeads) * ep.context * kHeadDim);
-#pragma unroll
-            for (int q = tid; q < BM * 16; q += kThreads) {
-                const int row = q >> 4, c8 = q & 15, m = m0 + row;
-                if (m < M)
-                    reinterpret_cast<u32x4*>(cache + size_t(ep.pos0 + m) * kHeadDim)[c8] =
-                        *reinterpret_cast<const u32x4*>(&ht[row][8 * c8]);
-            }
-        }
-    }
 }
 
 // x[b] = fp32(E[ids[b]]) (engine/core.cpp:382-383).
@@ -909,50 +425,69 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(float* __restrict__ X, c
     if (idx < size_t(rows) * kHidden) X[idx] = fold_splits<SPLITS>(X[idx], parts + idx, size_t(rows) * kHidden);
 }
 
-// The tallest tile (128, 64 or 32 rows) that still gives every CU a
-// workgroup; `splits` K ranges (EPI 2) count towards the workgroups.
+// Tiles: rows, outputs, MFMA wave grid (outputs x rows), LDS stages, stage depth.
+using Tile256 = GemmTile<128, 256, 4, 2, 2>;
+using Tile192 = GemmTile<128, 192, 2, 4, 2>;
+using Tile128 = GemmTile<128, 128, 2, 4, 3>;
+using Tile64 = GemmTile<64, 128, 4, 2, 5>;
+using Tile64n = GemmTile<64, 64, 2, 4, 6>;
+using Tile32 = GemmTile<32, 64, 2, 2, 8>;
+using Tile32n = GemmTile<32, 32, 1, 2, 6, 128>;
+using Tile16n = GemmTile<16, 32, 1, 1, 8>;
+using Qkv128 = GemmTile<128, 128, 1, 8, 3>;
+using Qkv64 = GemmTile<64, 128, 1, 4, 5>;
+using Qkv32 = GemmTile<32, 128, 1, 2, 6>;
+using Qkv16 = GemmTile<16, 128, 1, 1, 4, 128>;
+constexpr int kTileN = 128, kTileK = 64;  // N and K granularity of the GEMM entries
+
+template <class T, int EPI>
+void launch(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, int M, int N, int K,
+            hipStream_t stream, int splits, const GemmEpilogue& ep) {
+    gemm_kernel<T, EPI><<<dim3(GemmMap(M, N, T::BM, T::BN).groups(), 1, splits), T::kThreads, 0, stream>>>(
+        Ah, Al, W, C, M, N, K, ep);
+}
+
+// Every CU runs one workgroup at a time, so a launch takes as many rounds as
+// it has 256 workgroups; the tile with the least rounds x price is taken. A
+// price is the measured time of a round of that tile relative to 128 x 128
+// (20 us for gate/up: 16 x 32 7.0, 32 x 32 7.6, 32 x 64 8.3, 64 x 64 10.1,
+// 64 x 128 12.9, 128 x 192 28.5, 128 x 256 33; O and down within 10% of the same
+// ratios). Tiles of short prompts keep all CUs busy: one row tile of 128 x 128
+// would leave 208 of them idle in gate/up and run 19 us.
 template <int EPI>
 void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, int M, int N, int K,
           hipStream_t stream, int splits = 1, const GemmEpilogue& ep = {}) {
-    require(N % kTileN == 0 && K % (kTileK * splits) == 0 && M > 0 && (splits == 1 || EPI == 2),
+    require(N % kTileN == 0 && K % (kTileK * splits) == 0 && M > 0 &&
+                (splits == 1 || EPI == kParts || EPI == kPartsGuarded),
             "gemm: unsupported shape");
-    const int tiles = N / kTileN * splits;
-    auto launch = [&](auto bm, auto bn) {
-        constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value;
-        const int per = ((M + BM - 1) / BM + 7) / 8;  // row tiles per XCD
-        gemm_kernel<BM, EPI, BN><<<dim3(8 * per * (N / BN), 1, splits), GemmShape<BM, BN>::kWaves * 64, 0, stream>>>(
-            Ah, Al, W, C, M, N, K, ep);
-    };
-    using I128 = std::integral_constant<int, 128>;
-        // 128-row tiles of 128, 192 or 256 columns (the QKV epilogue takes one
-    // head per tile): the fewest rounds of 256 workgroups, each round priced
-    // at the measured time of one workgroup of that width relative to 128.
-    if constexpr (EPI != 4) {
-        const int mtiles = (M + 127) / 128;
-        auto cost = [&](int bn, double per_round) {
-            const long groups = long(mtiles) * (N / bn) * splits;
-            return (groups + 255) / 256 * per_round;
-        };
-        if (mtiles * tiles >= 256) {
-            const double c128 = cost(128, 1.0);
-            const double c192 = N % 192 == 0 ? cost(192, 1.45) : 1e30;
-            const double c256 = N % 256 == 0 ? cost(256, 1.91) : 1e30;
-            if (c256 <= c192 && c256 <= c128) {
-                launch(I128{}, std::integral_constant<int, 256>{});
-                return;
-            }
-            if (c192 <= c128) {
-                launch(I128{}, std::integral_constant<int, 192>{});
-                return;
-            }
+    double best = 1e30;
+    void (*run)(const uint16_t*, const uint16_t*, const uint16_t*, float*, int, int, int, hipStream_t, int,
+                const GemmEpilogue&) = nullptr;
+    auto consider = [&]<class T>(double price) {
+        if (N % T::BN != 0 || K % (T::TK * splits) != 0) return;
+        const long groups = long((M + T::BM - 1) / T::BM) * (N / T::BN) * splits;
+        const double cost = double((groups + 255) / 256) * price;
+        if (cost < best) {
+            best = cost;
+            run = &launch<T, EPI>;
         }
+    };
+    if constexpr (EPI == kQkv) {  // a head per tile; QKV rounds relative to Qkv128
+        consider.template operator()<Qkv16>(0.42);
+        consider.template operator()<Qkv32>(0.46);
+        consider.template operator()<Qkv64>(0.68);
+        consider.template operator()<Qkv128>(1.0);
+    } else {
+        consider.template operator()<Tile16n>(0.33);
+        consider.template operator()<Tile32n>(0.36);
+        consider.template operator()<Tile32>(0.40);
+        consider.template operator()<Tile64n>(0.49);
+        consider.template operator()<Tile64>(0.645);
+        consider.template operator()<Tile128>(1.0);
+        if constexpr (EPI != kParts && EPI != kPartsGuarded) consider.template operator()<Tile192>(1.44);
+        consider.template operator()<Tile256>(1.68);
     }
-    if ((M + 127) / 128 * tiles >= 256)
-        launch(I128{}, I128{});
-    else if ((M + 63) / 64 * tiles >= 256)
-        launch(std::integral_constant<int, 64>{}, I128{});
-    else
-        launch(std::integral_constant<int, 32>{}, I128{});
+    run(Ah, Al, W, C, M, N, K, stream, splits, ep);
 }
 
 // FP32 rows [M x K] -> FP16 hi / lo planes (GEMM operands handed over as
@@ -1005,10 +540,8 @@ void launch_gemm(const float* A, const uint16_t* W, float* C, int M, int N, int 
     with_planes(A, M, K, stream, [&](const uint16_t* hi, const uint16_t* lo, const int* row_exp) {
         GemmEpilogue ep{};
         ep.row_exp = row_exp;
-        if (accumulate)
-            gemm<1>(hi, lo, W, C, M, N, K, stream, 1, ep);
-        else
-            gemm<0>(hi, lo, W, C, M, N, K, stream, 1, ep);
+        ep.add = accumulate;
+        gemm<kStore>(hi, lo, W, C, M, N, K, stream, 1, ep);
     });
 }
 
@@ -1027,7 +560,7 @@ void launch_gemm_swiglu(const float* A, const uint16_t* W, uint16_t* act_hi, uin
         require(cleared == hipSuccess, "gemm swiglu: hipMemsetAsync failed");
         with_planes(A, M, K, stream, [&](const uint16_t* hi, const uint16_t* lo, const int* row_exp) {
             ep.row_exp = row_exp;
-            gemm<3>(hi, lo, W, nullptr, M, N, K, stream, 1, ep);
+            gemm<kSwiglu>(hi, lo, W, nullptr, M, N, K, stream, 1, ep);
         });
     } catch (...) {
         (void)hipFree(flags);
@@ -1073,10 +606,8 @@ void launch_gemm_static(const float* A, const uint16_t* W, float* C, int M, int 
     split_rows_kernel<<<M, 256, 0, stream>>>(A, hi, lo, row_exp, K);
     GemmEpilogue ep{};
     ep.row_exp = row_exp;
-    if (accumulate)
-        gemm<1>(hi, lo, W, C, M, N, K, stream, 1, ep);
-    else
-        gemm<0>(hi, lo, W, C, M, N, K, stream, 1, ep);
+    ep.add = accumulate;
+    gemm<kStore>(hi, lo, W, C, M, N, K, stream, 1, ep);
 }
 
 void launch_attention_prefill(const float* qkv, const uint16_t* keys, const uint16_t* values, uint16_t* att_hi,
@@ -1106,18 +637,18 @@ void launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, con
             rmsnorm_rows_kernel<kSplits><<<rows, 256, 0, stream>>>(s.x, L.in_norm, s.h_hi, s.h_lo, s.part, rows,
                                                                    s.row_exp, nullptr);
         GemmEpilogue ep{L.q_norm, L.k_norm, cosines, sines, L.keys, L.values, pos0, context, s.act_hi, s.act_lo,
-                        s.row_exp, s.act_flag, s.act_exp};
-        gemm<4>(s.h_hi, s.h_lo, L.qkv_n, s.qkv, rows, kQKVRows, kHidden, stream, 1, ep);
+                        s.row_exp, s.act_flag, s.act_exp, false};
+        gemm<kQkv>(s.h_hi, s.h_lo, L.qkv_n, s.qkv, rows, kQKVRows, kHidden, stream, 1, ep);
         launch_attention_prefill(s.qkv, L.keys, L.values, s.att_hi, s.att_lo, rows, pos0, context, stream);
         // The attention output is a convex combination of FP16 values: it fits FP16 unscaled.
-        gemm<2>(s.att_hi, s.att_lo, L.o_n, s.part, rows, kHidden, kQDim, stream, kSplits);
+        gemm<kParts>(s.att_hi, s.att_lo, L.o_n, s.part, rows, kHidden, kQDim, stream, kSplits);
         rmsnorm_rows_kernel<kSplits><<<rows, 256, 0, stream>>>(s.x, L.post_norm, s.h_hi, s.h_lo, s.part, rows,
                                                                s.row_exp, s.act_flag);
-        gemm<3>(s.h_hi, s.h_lo, L.gateup_n, nullptr, rows, 2 * kFFN, kHidden, stream, 1, ep);
+        gemm<kSwiglu>(s.h_hi, s.h_lo, L.gateup_n, nullptr, rows, 2 * kFFN, kHidden, stream, 1, ep);
         GemmEpilogue down{};
         down.act_flag = s.act_flag;
         down.act_exp = s.act_exp;
-        gemm<2>(s.act_hi, s.act_lo, L.down_n, s.part, rows, kHidden, kFFN, stream, kSplits, down);
+        gemm<kPartsGuarded>(s.act_hi, s.act_lo, L.down_n, s.part, rows, kHidden, kFFN, stream, kSplits, down);
     }
     fold_rows_kernel<kSplits><<<(rows * kHidden + 255) / 256, 256, 0, stream>>>(s.x, s.part, rows);
 }

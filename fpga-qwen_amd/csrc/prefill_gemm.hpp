@@ -1,0 +1,613 @@
+// The prefill GEMMs on the matrix cores: C[M x N] = A[M x K] . W[N x K]^T
+// with the layer work that follows each product in its epilogue.
+//
+// A arrives as two FP16 planes written by the kernel that produced it, hi =
+// fp16(a) and lo = fp16(a - hi) (a - hi is exact in FP32), W as its natural
+// FP16 rows; both planes are multiplied, so products are exact and sums FP32.
+//
+// Operand roles: W rows are the MFMA's A operand and activation rows its B
+// operand (v_mfma_f32_16x16x32_f16), so in the 16x16 result lane l holds
+// activation row l % 16 and, in its 4 registers, the 4 consecutive outputs
+// 4 (l / 16) .. + 3. A wave therefore has whole pieces of a row's outputs in
+// its registers, and the epilogues (QK-norm, RoPE, SwiGLU, splits) run there,
+// without staging C in LDS: a row sum is an in-lane sum plus exchanges with
+// lanes l ^ 16 and l ^ 32.
+//
+// Each output element adds its K terms in one order whatever the tile: steps
+// of 32 in ascending k, hi then lo in each. Results do not depend on M, on a
+// row's place in a tile or on the tile shape.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "half_split.hpp"
+#include "kernels.hpp"
+#include "prefill.hpp"
+
+namespace qwen_hip {
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane from global memory straight into LDS at
+// lds + 16 lane (lds wave-uniform); counted by vmcnt like any load.
+__device__ __forceinline__ void load_lds16(const void* src, unsigned char* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
+#endif
+}
+
+// vmcnt <= n (expcnt and lgkmcnt unconstrained).
+template <int n>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(n >= 0 && n < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// lgkmcnt == 0 (this wave's LDS accesses have completed).
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
+
+// Workgroup barrier without a memory fence: the waits before it already
+// cover the direct-to-LDS loads (a fenced barrier would wait for every load
+// in flight, including the later stages). The empty asm statements keep the
+// compiler from moving LDS accesses across it.
+__device__ __forceinline__ void stage_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// v of lane ^ 16 and of lane ^ 32, through the row swaps (register speed).
+__device__ __forceinline__ int lane_xor16(int v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return int((threadIdx.x & 16) ? r[0] : r[1]);
+}
+__device__ __forceinline__ int lane_xor32(int v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return int((threadIdx.x & 32) ? r[0] : r[1]);
+}
+__device__ __forceinline__ float lane_xor16(float v) { return __int_as_float(lane_xor16(__float_as_int(v))); }
+__device__ __forceinline__ double lane_xor16(double v) {
+    return __hiloint2double(lane_xor16(__double2hiint(v)), lane_xor16(__double2loint(v)));
+}
+__device__ __forceinline__ double lane_xor32(double v) {
+    return __hiloint2double(lane_xor32(__double2hiint(v)), lane_xor32(__double2loint(v)));
+}
+
+enum GemmKind { kStore, kParts, kPartsGuarded, kSwiglu, kQkv };
+
+// Work fused into the epilogue. QKV (kQkv): QK-norm, RoPE and the K/V cache
+// writes of engine/core.cpp:395-406. Gate/up (kSwiglu): SwiGLU, written as
+// the FP16 hi / lo planes the down GEMM reads.
+//
+// Range guard of the FP16 split (split_exponent): A row m that its producer
+// split as a * 2^-row_exp[m] has its products scaled back by 2^row_exp[m]
+// (kStore, kSwiglu, kQkv). The SwiGLU
+// epilogue splits each group of 8 activations with its own exponent, stored
+// in act_exp [M][N / 16], and raises act_flag [M][4] (one word per K range of
+// the down GEMM, cleared by the kernel before the gate/up GEMM) to the
+// largest exponent in the range. The down GEMM (kParts with act_flag) runs
+// its plain K loop, and a workgroup whose rows saw a nonzero flag runs the
+// loop again with every group rescaled in LDS to its row's flag exponent
+// and the products scaled back: a row that fits keeps its bits.
+struct GemmEpilogue {
+    const float* q_norm;
+    const float* k_norm;
+    const float* cosines;
+    const float* sines;
+    uint16_t* keys;
+    uint16_t* values;
+    int pos0;
+    int context;
+    uint16_t* act_hi;
+    uint16_t* act_lo;
+    const int* row_exp;
+    int* act_flag;
+    uint8_t* act_exp;
+    bool add;  // kStore: C += instead of C =
+};
+
+// Tile of a workgroup: BM activation rows x BN outputs, K in stages of TK
+// through a ring of NS LDS buffers. WN x WM waves run the MFMAs: wave (wn, wm)
+// holds the 16-output tiles wn TN .. and the 16-row tiles wm TM ... 4 more
+// waves, one per SIMD, only issue the direct global -> LDS loads: a CU accepts
+// 64 bytes of loads per clock, so a stage's loads hold up the waves that issue
+// them for about as long as the stage's MFMAs take, and waves that do both can
+// do neither during the other.
+template <int BM_, int BN_, int WN_, int WM_, int NS_, int TK_ = 64>
+struct GemmTile {
+    static constexpr int BM = BM_, BN = BN_, WN = WN_, WM = WM_, NS = NS_, TK = TK_;
+    static constexpr int kMma = WN * WM, kLoaders = 4, kThreads = 64 * (kMma + kLoaders);
+    static constexpr int TN = BN / 16 / WN, TM = BM / 16 / WM;  // 16x16 result tiles per MFMA wave
+    static constexpr int SL = TK / 8;                           // 16-byte slots per operand row
+    static constexpr int kSubs = TK / 32;                       // 32-column steps per stage
+    static constexpr int kPlane = BM * SL, kSlots = 2 * kPlane + BN * SL;
+    static constexpr int kStageBytes = 16 * kSlots;
+    static constexpr int kLoads = kSlots / 64 / kLoaders;       // 1 KiB loads per loader and stage
+    // Stages sent off before the first wait: 48 KiB or more, so that the first
+    // one does not queue behind a whole ring.
+    static constexpr int kFirst = kStageBytes >= 48 * 1024 ? 1 : (48 * 1024 + kStageBytes - 1) / kStageBytes;
+    static_assert(kMma <= 8 && TN * WN * 16 == BN && TM * WM * 16 == BM, "wave grid");
+    static_assert(kLoads * 64 * kLoaders == kSlots && kPlane % 64 == 0, "every loader issues the same number of loads");
+    static_assert((TK == 64 || TK == 128) && NS >= 2 && NS * kStageBytes <= 160 * 1024 && (NS - 1) * kLoads < 64,
+                  "stages");
+};
+
+// LDS operand rows of TK halves: piece p of row r sits in 16-byte slot
+// SL r + (p ^ swz(r)), so that the 16 rows read at one piece by the lanes of
+// a 16-lane group fill the 16 slots of a 256-byte bank cycle.
+template <int TK>
+__device__ __forceinline__ int gemm_swz(int r) {
+    return TK == 64 ? ((r >> 1) ^ ((r & 1) << 2)) & 7 : r & 15;
+}
+
+// Tile order. Workgroup w runs on XCD w % 8 (round-robin dispatch). The XCDs
+// form 8 / f groups of f: group i takes the row tiles i, i + 8 / f, ... and its
+// XCDs split the column tiles by residue mod f, so each W tile is fetched by
+// 8 / f XCDs and each A row by f. Short prompts (few row tiles) are bound by
+// the weights: every W tile goes to one XCD (f = 8). With 4 or more row tiles
+// per XCD its 32 CUs share rows and columns within the L2 at f = 1.
+struct GemmMap {
+    int mtiles, ntiles, f, per;  // per: row tiles of a group
+    __host__ __device__ GemmMap(int M, int N, int BM, int BN) {
+        mtiles = (M + BM - 1) / BM;
+        ntiles = N / BN;
+        f = mtiles <= 4 ? 8 : mtiles <= 8 ? 4 : mtiles < 25 ? 2 : 1;
+        per = (mtiles + 8 / f - 1) / (8 / f);
+    }
+    __host__ __device__ int groups() const { return 8 * per * ((ntiles + f - 1) / f); }
+};
+
+// gate * sigmoid(gate) * up with sigmoid(g) = 0.5 + 0.5 tanh(g / 2)
+// (engine/core.cpp:636-639) from one exp2 and one correctly rounded division:
+// within 2 ulp of the exact sigmoid where it is not tiny, and exp2's argument
+// rounding (2^-24 |g|, relative) where it is, against the 2^-25 absolute of
+// the tanh form.
+__device__ __forceinline__ float swiglu(float gate, float up) {
+    const float sig = 1.0f / (1.0f + __builtin_amdgcn_exp2f(gate * -1.4426950408889634f));
+    return gate * sig * up;
+}
+
+template <class T, int EPI>
+__global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __restrict__ Ah,
+                                                           const uint16_t* __restrict__ Al,
+                                                           const uint16_t* __restrict__ W, float* __restrict__ C, int M,
+                                                           int N, int K, GemmEpilogue ep) {
+    constexpr int BM = T::BM, BN = T::BN, WN = T::WN, TN = T::TN, TM = T::TM, NS = T::NS, TK = T::TK, SL = T::SL;
+    constexpr int kLoads = T::kLoads, kStageBytes = T::kStageBytes, kPlane = T::kPlane;
+    static_assert(EPI != kQkv || (WN == 1 && BN == kHeadDim), "a wave of the QKV epilogue holds whole heads");
+    static_assert(EPI != kSwiglu || TN % 2 == 0, "a wave of the SwiGLU epilogue holds gate and up tiles");
+    // Results staged for the stores, over the ring: QKV rows of a wave, the
+    // SwiGLU planes or the C tile of the workgroup; pitches 16 bytes past a
+    // multiple of the banks.
+    constexpr int kPitch = EPI == kQkv ? 4 * kHeadDim + 16 : EPI == kSwiglu ? BN + 16 : 4 * BN + 16;  // bytes
+    constexpr int kOutBytes = EPI == kQkv ? T::kMma * 16 * kPitch : EPI == kSwiglu ? 2 * BM * kPitch : BM * kPitch;
+    constexpr int kSmem = NS * kStageBytes > kOutBytes ? NS * kStageBytes : kOutBytes;
+    static_assert(kSmem <= 160 * 1024, "LDS");
+    __shared__ __align__(16) unsigned char smem[kSmem];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const GemmMap map(M, N, BM, BN);
+    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, groups = 8 / map.f;
+    const int mt = xcd / map.f + groups * (slot % map.per), nt = xcd % map.f + map.f * (slot / map.per);
+    if (mt >= map.mtiles || nt >= map.ntiles) return;
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool mma = wave < T::kMma;
+    const int wn = wave % WN, wm = wave / WN % T::WM;
+    const int ks = K / gridDim.z, kz = blockIdx.z * ks, nk = ks / TK;  // this workgroup's K range
+    const int row = lane & 15, quad = lane >> 4;  // result row and output group of this lane
+
+    // Loader i's load j fills slots 64 (i + 4 j) + lane of a stage: A hi, A lo,
+    // then W rows; 64 / SL rows each. A rows past M repeat row M - 1 and are
+    // never stored.
+    const char* base[kLoads];   // wave-uniform
+    unsigned offset[kLoads];
+    auto load_addresses = [&] {
+        const int loader = wave - T::kMma;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int q0 = 64 * (loader + T::kLoaders * j);
+            const bool is_w = q0 >= 2 * kPlane;
+            const int r = (q0 - (is_w ? 2 * kPlane : q0 >= kPlane ? kPlane : 0)) / SL + lane / SL;
+            const int p = (lane % SL) ^ gemm_swz<TK>(r);
+            if (is_w) {
+                const int r0 = r - lane / SL;
+                const int first = EPI == kSwiglu ? (r0 < BN / 2 ? n0 / 2 : N / 2 + n0 / 2 - BN / 2) : n0;
+                base[j] = reinterpret_cast<const char*>(W + size_t(first) * K + kz);
+                offset[j] = 2u * (unsigned(r) * unsigned(K) + 8u * p);
+            } else {
+                base[j] = reinterpret_cast<const char*>((q0 >= kPlane ? Al : Ah) + size_t(m0) * K + kz);
+                offset[j] = 2u * (unsigned(min(r, M - 1 - m0)) * unsigned(K) + 8u * p);
+            }
+        }
+    };
+    auto issue = [&](int kt) {
+        unsigned char* stage = smem + (kt % NS) * kStageBytes + 1024 * (wave - T::kMma);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j)
+            load_lds16(base[j] + offset[j] + kt * TK * 2, stage + 1024 * T::kLoaders * j);
+    };
+    // Waits until at most `later` whole stages of this loader's are pending.
+    auto wait_stages = [&](int later) {
+        if (later >= NS - 1) {
+            wait_vmcnt<(NS - 1) * kLoads>();
+        } else {
+            switch (later) {
+                case 0: wait_vmcnt<0>(); break;
+                case 1: wait_vmcnt<(NS > 2 ? 1 : 0) * kLoads>(); break;
+                case 2: wait_vmcnt<(NS > 3 ? 2 : 0) * kLoads>(); break;
+                case 3: wait_vmcnt<(NS > 4 ? 3 : 0) * kLoads>(); break;
+                case 4: wait_vmcnt<(NS > 5 ? 4 : 0) * kLoads>(); break;
+                case 5: wait_vmcnt<(NS > 6 ? 5 : 0) * kLoads>(); break;
+                default: wait_vmcnt<(NS > 7 ? 6 : 0) * kLoads>(); break;
+            }
+        }
+    };
+
+    int flag0 = 0, flag1 = 0;  // range flags of the workgroup's rows, read by every wave
+    if constexpr (EPI == kPartsGuarded) {
+        flag0 = ep.act_flag[size_t(min(m0 + lane % BM, M - 1)) * 4 + blockIdx.z];
+        if constexpr (BM > 64) flag1 = ep.act_flag[size_t(min(m0 + 64 + lane, M - 1)) * 4 + blockIdx.z];
+    }
+
+    floatx4 acc[TN][TM];
+    auto clear = [&] {
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int t = 0; t < TM; ++t) acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    // Operands of MFMA step `sub` of a stage: lane l reads k = 32 sub +
+    // 8 (l / 16) .. + 7 of row l % 16 of each tile (tile offsets are
+    // immediates: the swizzle depends on the row mod 16 only).
+    auto operand_base = [&](const unsigned char* stage, int sub) {
+        return stage + 16 * (SL * row + ((4 * sub + quad) ^ gemm_swz<TK>(row)));
+    };
+    // Output tile i of this wave starts at W row w_row(i) of the tile: gate
+    // tiles then their up tiles (SwiGLU), else in order.
+    auto w_row = [&](int i) {
+        if constexpr (EPI == kSwiglu) return 16 * (wn * (TN / 2) + i % (TN / 2)) + (i < TN / 2 ? 0 : BN / 2);
+        return 16 * (wn * TN + i);
+    };
+    auto read_w = [&](const unsigned char* at, int i) {
+        return *reinterpret_cast<const half8*>(at + 32 * kPlane + 16 * SL * w_row(i));
+    };
+    auto read_a = [&](const unsigned char* at, int plane, int t) {
+        return *reinterpret_cast<const half8*>(at + 16 * kPlane * plane + 256 * SL * (wm * TM + t));
+    };
+    // Half of a step: the products of one A plane, with side(c) behind MFMA c.
+    auto multiply = [&](const half8 (&w)[TN], const half8 (&a)[TM], auto&& side) {
+#pragma unroll
+        for (int c = 0; c < TM * TN; ++c) {
+            const int i = c % TN, t = c / TN;
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[i], a[t], acc[i][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            side(c);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    int rexp[TM];
+    if (!mma) {
+        // Loaders: stage kt is handed over by barrier kt, behind which the MFMA
+        // waves have read stage kt - 1 and its buffer is refilled.
+        load_addresses();
+        int sent = 0;
+        for (; sent < min(T::kFirst, nk); ++sent) issue(sent);
+        for (int kt = 0; kt < nk; ++kt) {
+            // Behind barrier kt the buffer of stage kt - 1 is free.
+            if (kt == 0 && sent < nk && T::kFirst < NS) issue(sent++);
+            wait_stages(sent - kt - 1);  // stage kt has landed
+            stage_barrier();
+#pragma unroll
+            for (int more = 0; more < 2; ++more)
+                if (sent < min(nk, kt + NS)) issue(sent++);
+        }
+    } else {
+        // MFMA waves: the second half of a step reads the next step's W and A
+        // hi operands, the first half its own A lo, one read behind each of
+        // its first MFMAs. The barrier that hands over the next stage comes
+        // between the halves of a stage's last step, when every operand of the
+        // stage is in registers.
+        if constexpr (EPI != kParts && EPI != kPartsGuarded) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) rexp[t] = ep.row_exp[min(m0 + (wm * TM + t) * 16 + row, M - 1)];
+        }
+        clear();
+        half8 w[2][TN], h[TM], l[TM];
+        stage_barrier();
+        {
+            const unsigned char* at = operand_base(smem, 0);
+#pragma unroll
+            for (int i = 0; i < TN; ++i) w[0][i] = read_w(at, i);
+#pragma unroll
+            for (int t = 0; t < TM; ++t) h[t] = read_a(at, 0, t);
+        }
+        for (int kt = 0; kt < nk; ++kt) {
+            const unsigned char* stage = smem + (kt % NS) * kStageBytes;
+#pragma unroll
+            for (int sub = 0; sub < T::kSubs; ++sub) {
+                const unsigned char* at = operand_base(stage, sub);
+                wait_lgkm0();
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(w[sub & 1], h, [&](int c) {
+                    if (c < TM) l[c] = read_a(at, 1, c);
+                });
+                wait_lgkm0();
+                const unsigned char* next = operand_base(stage, sub + 1);
+                if (sub + 1 == T::kSubs) {
+                    next = operand_base(smem + ((kt + 1) % NS) * kStageBytes, 0);
+                    if (kt + 1 < nk) stage_barrier();
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                // The reads behind the range's last step fetch a stage that is
+                // not there: in bounds of the ring, never used.
+                multiply(w[sub & 1], l, [&](int c) {
+                    constexpr int kReads = TN + TM, kPer = (kReads + TM * TN - 1) / (TM * TN);
+#pragma unroll
+                    for (int r = c * kPer; r < (c + 1) * kPer; ++r) {
+                        if (r < TM) h[r] = read_a(next, 0, r);
+                        else if (r < kReads) w[(sub + 1) & 1][r - TM] = read_w(next, r - TM);
+                    }
+                });
+            }
+        }
+        wait_lgkm0();
+    }
+
+    // Guarded down GEMM: the loop again with each A group rescaled in LDS to its
+    // row's flag exponent (exact: FP16 values times powers of two no greater
+    // than 1), one stage at a time. Every wave read the same flags, so every
+    // wave takes the same branch.
+    bool rescaled = false;
+    if constexpr (EPI == kPartsGuarded) {
+        if (__builtin_amdgcn_ballot_w64(flag0 != 0 || flag1 != 0) != 0) {
+            rescaled = true;
+            clear();
+            for (int kt = 0; kt < nk; ++kt) {
+                stage_barrier();  // every wave is done with the stage before (all loads were waited for)
+                unsigned char* stage = smem + (kt % NS) * kStageBytes;
+                if (!mma) {
+                    issue(kt);
+                    wait_vmcnt<0>();
+                }
+                stage_barrier();
+                for (int q = tid; q < kPlane; q += T::kThreads) {
+                    const int r = q / SL, p = (q % SL) ^ gemm_swz<TK>(r), m = min(m0 + r, M - 1);
+                    const int er = ep.act_flag[size_t(m) * 4 + blockIdx.z];
+                    if (er != 0) {
+                        const int e8 = ep.act_exp[size_t(m) * (K / 8) + (kz + kt * TK) / 8 + p];
+                        const float sc = pow2(e8 - er);
+                        half8* hp = reinterpret_cast<half8*>(stage + 16 * q);
+                        half8* lp = reinterpret_cast<half8*>(stage + 16 * (kPlane + q));
+                        half8 hv = *hp, lv = *lp;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            hv[e] = static_cast<_Float16>(static_cast<float>(hv[e]) * sc);
+                            lv[e] = static_cast<_Float16>(static_cast<float>(lv[e]) * sc);
+                        }
+                        *hp = hv;
+                        *lp = lv;
+                    }
+                }
+                wait_lgkm0();
+                stage_barrier();
+                if (mma) {
+#pragma unroll
+                    for (int sub = 0; sub < T::kSubs; ++sub) {
+                        const unsigned char* at = operand_base(stage, sub);
+                        half8 w[TN], h[TM], l[TM];
+#pragma unroll
+                        for (int i = 0; i < TN; ++i) w[i] = read_w(at, i);
+#pragma unroll
+                        for (int t = 0; t < TM; ++t) {
+                            h[t] = read_a(at, 0, t);
+                            l[t] = read_a(at, 1, t);
+                        }
+                        multiply(w, h, [](int) {});
+                        multiply(w, l, [](int) {});
+                    }
+                    wait_lgkm0();
+                }
+            }
+        }
+    }
+    stage_barrier();  // every wave is done with the ring: the results are staged over it
+
+    if constexpr (EPI <= kPartsGuarded) {
+        if (mma) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+                const int r = (wm * TM + t) * 16 + row;
+                float sc = 1.f;
+                if constexpr (EPI == kPartsGuarded) {
+                    if (rescaled) sc = pow2(ep.act_flag[size_t(min(m0 + r, M - 1)) * 4 + blockIdx.z]);
+                } else if constexpr (EPI == kStore) {
+                    sc = pow2(rexp[t]);
+                }
+#pragma unroll
+                for (int i = 0; i < TN; ++i) {
+                    floatx4 v = acc[i][t];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] *= sc;
+                    *reinterpret_cast<floatx4*>(smem + r * kPitch + 4 * (w_row(i) + 4 * quad)) = v;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int q = tid; q < BM * (BN / 4); q += T::kThreads) {
+            const int r = q / (BN / 4), c4 = q % (BN / 4), m = m0 + r;
+            if (m < M) {
+                floatx4 v = *reinterpret_cast<const floatx4*>(smem + r * kPitch + 16 * c4);
+                floatx4* c = reinterpret_cast<floatx4*>(C + (size_t(blockIdx.z) * M + m) * N + n0) + c4;
+                if constexpr (EPI == kStore) {
+                    if (ep.add) {
+                        const floatx4 o = *c;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = o[e] + v[e];
+                    }
+                }
+                *c = v;
+            }
+        }
+    } else if constexpr (EPI == kSwiglu) {
+        // Gate tiles i < TN / 2, their up tiles i + TN / 2. Lanes l and l ^ 16
+        // hold a group of 8 activations: its largest magnitude sets the
+        // group's exponent, and the range's flag holds the largest of those.
+        if (mma) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+                const int r = (wm * TM + t) * 16 + row, m = m0 + r;
+                const float sc = pow2(rexp[t]);
+#pragma unroll
+                for (int i = 0; i < TN / 2; ++i) {
+                    float o[4], big = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        o[e] = swiglu(acc[i][t][e] * sc, acc[i + TN / 2][t][e] * sc);
+                        big = fmaxf(big, fabsf(o[e]));
+                    }
+                    big = fmaxf(big, lane_xor16(big));
+                    const int e8 = split_exponent(big), col = w_row(i) + 4 * quad;
+                    const float down = pow2(-e8);
+                    half4 hi, lo;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        _Float16 h, l;
+                        split_half(o[e] * down, h, l);
+                        hi[e] = h;
+                        lo[e] = l;
+                    }
+                    *reinterpret_cast<half4*>(smem + r * kPitch + 2 * col) = hi;
+                    *reinterpret_cast<half4*>(smem + (BM + r) * kPitch + 2 * col) = lo;
+                    if (m < M && (quad & 1) == 0) {
+                        const int at = n0 / 2 + col;
+                        ep.act_exp[size_t(m) * (N / 16) + at / 8] = static_cast<uint8_t>(e8);
+                        if (e8 != 0) atomicMax(ep.act_flag + size_t(m) * 4 + at / (N / 8), e8);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int q = tid; q < 2 * BM * (BN / 16); q += T::kThreads) {
+            const int rp = q / (BN / 16), c8 = q % (BN / 16), m = m0 + rp % BM;
+            if (m < M) {
+                uint16_t* plane = rp < BM ? ep.act_hi : ep.act_lo;
+                *reinterpret_cast<u32x4*>(plane + size_t(m) * (N / 2) + n0 / 2 + 8 * c8) =
+                    *reinterpret_cast<const u32x4*>(smem + rp * kPitch + 16 * c8);
+            }
+        }
+    } else if (mma) {
+        // Head nt of rows m: this lane holds channels j = 16 i + 4 quad + e
+        // (i < 8, e < 4), so the RoPE pair (j, j + 64) is in tiles i and i + 4.
+        const int head = nt;
+        const bool is_q = head < kQHeads, is_v = head >= kQHeads + kKVHeads;
+        unsigned char* out = smem + wave * 16 * kPitch;  // this wave's rows
+#pragma unroll
+        for (int t = 0; t < TM; ++t) {
+            const int mw = m0 + (wm * TM + t) * 16, m = mw + row;
+            const float sc = pow2(rexp[t]);
+            float x[8][4];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[i][e] = acc[i][t][e] * sc;
+            if (is_v) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    half4 hv;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) hv[e] = to_half(x[i][e]);
+                    *reinterpret_cast<half4*>(out + row * kPitch + 2 * (16 * i + 4 * quad)) = hv;
+                }
+            } else {
+                double sum = 0.0;  // FP32 squares, FP64 sum (engine/core.cpp:207-215)
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float square = x[i][e] * x[i][e];
+                        sum += static_cast<double>(square);
+                    }
+                sum += lane_xor16(sum);
+                sum += lane_xor32(sum);
+                const float inv = 1.0f / __builtin_sqrtf(static_cast<float>(sum) / 128.0f + 1e-6f);
+                const float* nw = (is_q ? ep.q_norm : ep.k_norm) + 4 * quad;
+                const size_t rope = size_t(ep.pos0 + min(m, M - 1)) * 64 + 4 * quad;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const floatx4 w0 = *reinterpret_cast<const floatx4*>(nw + 16 * i);
+                    const floatx4 w1 = *reinterpret_cast<const floatx4*>(nw + 16 * i + 64);
+                    const floatx4 cs = *reinterpret_cast<const floatx4*>(ep.cosines + rope + 16 * i);
+                    const floatx4 sn = *reinterpret_cast<const floatx4*>(ep.sines + rope + 16 * i);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float a = (x[i][e] * inv) * w0[e], b = (x[i + 4][e] * inv) * w1[e];
+                        x[i][e] = a * cs[e] - b * sn[e];
+                        x[i + 4][e] = b * cs[e] + a * sn[e];
+                    }
+                }
+                // Chain-permuted order (kperm): channel j = 8 s + c has its
+                // place in piece c + 8 (s / 8) at s % 8. This lane holds
+                // c = 4 (quad & 1) + e and s = 2 i + quad / 2, lane ^ 32 the
+                // other parity of s; trading the tiles i >= 4 of the lower half
+                // of the lanes for the tiles i < 4 of the upper half leaves lane
+                // half `up` with all 8 steps of the pieces c + 8 up.
+                const int piece = 4 * (quad & 1) + 8 * (lane >> 5);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float y[8];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x[i][e]),
+                                                                        __float_as_int(x[i + 4][e]), false, false);
+                        y[2 * i] = __int_as_float(int(r[0]));
+                        y[2 * i + 1] = __int_as_float(int(r[1]));
+                    }
+                    if (is_q) {
+                        floatx4* q = reinterpret_cast<floatx4*>(out + row * kPitch + 32 * (piece + e));
+                        q[0] = floatx4{y[0], y[1], y[2], y[3]};
+                        q[1] = floatx4{y[4], y[5], y[6], y[7]};
+                    } else {
+                        half8 hv;
+#pragma unroll
+                        for (int s = 0; s < 8; ++s) hv[s] = to_half(y[s]);
+                        *reinterpret_cast<half8*>(out + row * kPitch + 16 * (piece + e)) = hv;
+                    }
+                }
+            }
+            // The rows are this wave's own: whole rows out, 16 bytes per lane.
+            wait_lgkm0();
+            asm volatile("" ::: "memory");
+            if (is_q) {
+#pragma unroll 4
+                for (int q = lane; q < 16 * 32; q += 64) {
+                    const int r = q >> 5, c4 = q & 31;
+                    if (mw + r < M)
+                        reinterpret_cast<floatx4*>(C + size_t(mw + r) * N + head * kHeadDim)[c4] =
+                            *reinterpret_cast<const floatx4*>(out + r * kPitch + 16 * c4);
+                }
+            } else {
+                uint16_t* cache = is_v ? ep.values + size_t(head - kQHeads - kKVHeads) * ep.context * kHeadDim
+                                       : ep.keys + size_t(head - kQHeads) * ep.context * kHeadDim;
+#pragma unroll
+                for (int q = lane; q < 16 * 16; q += 64) {
+                    const int r = q >> 4, c8 = q & 15;
+                    if (mw + r < M)
+                        reinterpret_cast<u32x4*>(cache + size_t(ep.pos0 + mw + r) * kHeadDim)[c8] =
+                            *reinterpret_cast<const u32x4*>(out + r * kPitch + 16 * c8);
+                }
+            }
+            wait_lgkm0();
+            asm volatile("" ::: "memory");
+        }
+    }
+}
+
+}  // namespace
+}  // namespace qwen_hip

@@ -271,3 +271,58 @@ def test_prefill_rows_independent_of_grouping(qpkg, pack0):
         m.prefill(prompt[:1024])
         m.step(prompt[1024])
         assert np.array_equal(m.logits().view(np.uint32), tail)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n,k', [(1024, 1024), (4096, 1024), (1024, 3072), (6144, 64)])
+def test_gemm_tile_edges(qpkg, n, k):
+    """Row counts at the edges of every tile height (16, 32, 64, 128) and of
+    the rounds that choose between them: each call's rows must be the bits of
+    one 700-row call (whatever tile either takes, every element adds its K
+    terms in one order), which in turn meets the FP64 bound. K = 64 is a
+    single LDS stage."""
+    rng = np.random.default_rng(n + k)
+    a = rng.standard_normal((700, k), dtype=np.float32)
+    w = (rng.standard_normal((n, k), dtype=np.float32) * 0.02).astype(np.float16)
+    full = qpkg.gemm(a, w)
+    bound = 4e-6 * (np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T) + 1e-7
+    assert np.all(np.abs(full - a.astype(np.float64) @ w.astype(np.float64).T) <= bound)
+    for m in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 513):
+        first = (37 * m) % (700 - m)
+        got = qpkg.gemm(a[first:first + m], w)
+        assert np.array_equal(got.view(np.uint32), full[first:first + m].view(np.uint32)), m
+
+
+@pytest.mark.gpu
+def test_gemm_swiglu_tile_edges(qpkg):
+    """The same for the SwiGLU epilogue (gate and up columns of one tile), with
+    rows whose activations carry exponents among them."""
+    rng = np.random.default_rng(61)
+    a = rng.standard_normal((1300, 1024), dtype=np.float32)
+    a[::5] *= np.float32(300)
+    w = (rng.standard_normal((6144, 1024), dtype=np.float32) * 0.02).astype(np.float16)
+    full, exps = qpkg.gemm_swiglu(a, w, exponents=True)
+    assert exps.any() and not exps.all() and np.isfinite(full).all()
+    for m in (1, 16, 17, 32, 33, 64, 65, 128, 129, 320, 321, 640, 641, 1024, 1025):
+        first = (37 * m) % (1300 - m)
+        got, e = qpkg.gemm_swiglu(a[first:first + m], w, exponents=True)
+        assert np.array_equal(got.view(np.uint32), full[first:first + m].view(np.uint32)), m
+        assert np.array_equal(e, exps[first:first + m]), m
+
+
+@pytest.mark.gpu
+def test_prefill_rows_independent_of_tile(qpkg, pack0):
+    """The QKV epilogue (a head per tile of 16, 32, 64 or 128 rows) and the
+    K-split GEMMs: calls of 2 to 300 rows leave the logits of one 700-row
+    call."""
+    prompt = PROMPTS['long_3968'][:700]
+    with qpkg.Model(pack0) as m:
+        m.prefill(prompt)
+        whole = m.logits().view(np.uint32).copy()
+        m.reset()
+        at = 0
+        for rows in (2, 16, 17, 33, 65, 130, 137, 300):
+            m.prefill(prompt[at:at + rows])
+            at += rows
+        assert at == 700
+        assert np.array_equal(m.logits().view(np.uint32), whole)
