@@ -147,19 +147,22 @@ constexpr float kFaLazyMax = 8.f;
 // Workgroup = 32 consecutive query rows x one KV head g, 8 waves: wave
 // (h, s) = (wave & 1, wave >> 1) runs query head 2g + h over the key tiles
 // kt = s (mod 4) with its own online softmax, and the 4 key splits of each
-// head are merged at the end. The two waves of a split use the same tiles:
-// they load each K/V tile together (direct global -> LDS loads, 8 KiB each)
-// into a double-buffered LDS ring, one tile ahead of the matrix cores, so a
-// wave streams half a tile per step instead of a whole one (a wave retires
-// only about 10 GB/s of loads). K is read from LDS as the S^T operand and V^T
-// with the LDS transpose load (ds_read_b64_tr_b16), so V needs no transpose
-// pass through registers.
+// head are merged at the end. The two waves of a split load its K and V tiles
+// together (direct global -> LDS loads, two buffers of each).
+//
+// A step of a wave is a matrix phase (P V of its last tile, then K Q of the
+// next) and a vector phase (loads of later tiles, softmax). The two waves of a
+// SIMD (splits s and s + 2) run them alternately, one barrier per phase: while
+// one multiplies, the other exponentiates. With both in the same phase a step
+// took 3,700 clocks (at 2,100 of MFMAs per SIMD), the vector work and the
+// acceptance of 64 KiB of loads (700 clocks) serial with the MFMAs.
 constexpr int kFbTileBytes = kFaKeys * kHeadDim * 2;        // one K or V tile (8 KiB)
-constexpr int kFbSplitBytes = 2 * kFbTileBytes;             // K then V of one split
-constexpr int kFbStageBytes = 4 * kFbSplitBytes;            // the 4 splits' tiles of one step
+constexpr int kFbSplitBytes = 4 * kFbTileBytes;             // a split's K buffers 0 and 1, then its V buffers
 constexpr int kFbMergeBytes = 8 * kFaRows * kFaccPitch * 4; // 8 waves' outputs
-constexpr int kFbLds = 2 * kFbStageBytes > kFbMergeBytes ? 2 * kFbStageBytes : kFbMergeBytes;
+constexpr int kFbLds = 4 * kFbSplitBytes > kFbMergeBytes ? 4 * kFbSplitBytes : kFbMergeBytes;
 typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 // K and V tiles in LDS: rows of 128 halves (sixteen 16-byte pieces), piece p
 // of key row r in 16-byte slot 16 r + (p ^ fb_swz(r)). fb_swz is a bijection
@@ -173,14 +176,47 @@ __device__ __forceinline__ int fb_slot(int r, int p) { return 16 * r + (p ^ fb_s
 // ds_read_b64_tr_b16 (gfx950): within each 16-lane group, lane 4a + b
 // receives element b of the 8-byte chunks addressed by lanes a, a + 4,
 // a + 8 and a + 12, in that order.
-__device__ __forceinline__ short4_t lds_read_tr16(const unsigned char* p) {
+__device__ __forceinline__ short4_t lds_read_tr16(unsigned address) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) short4_t*)(const_cast<unsigned char*>(p)));
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(address));
 #else
-    (void)p;
+    (void)address;
     return short4_t{0, 0, 0, 0};
 #endif
+}
+__device__ __forceinline__ half8 lds_read16(unsigned address) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return *(__attribute__((address_space(3))) const half8*)(address);
+#else
+    (void)address;
+    return half8{};
+#endif
+}
+
+// v - float(h[E]), exact where h[E] is v rounded: one mixed-precision FMA.
+template <int E>
+__device__ __forceinline__ float rest_of_half(half2 h, float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    if constexpr (E == 0)
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    else
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(v));
+    return r;
+#else
+    return v - static_cast<float>(h[E]);
+#endif
+}
+
+// Largest value of the 8 lanes of an aligned group.
+__device__ __forceinline__ float max_of_8(float v) {
+    auto dpp = [](float x, auto ctrl) {
+        const int b = __float_as_int(x);
+        return __int_as_float(__builtin_amdgcn_update_dpp(b, b, decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v = fmaxf(v, dpp(v, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp(v, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
+    return fmaxf(v, dpp(v, std::integral_constant<int, 0x141>{}));  // the other quad of 8 lanes
 }
 
 __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __restrict__ QKV,
@@ -191,13 +227,15 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
                                                                   int context, float scale) {
     __shared__ __align__(16) unsigned char lds[kFbLds];
     __shared__ float fm[8][kFaRows], fl[8][kFaRows];
+    __shared__ int q_exp[2][kFaRows];
     // Workgroup w runs on XCD w % 8 (round-robin dispatch): KV head g = w % 8
     // keeps every workgroup reading one head's K/V rows on one XCD, so they
     // stay in its L2; the query blocks run heaviest (latest) first.
     const int nqb = gridDim.x / kKVHeads;
     const int g = blockIdx.x % kKVHeads, qb = nqb - 1 - blockIdx.x / kKVHeads;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h = wave & 1, sp = wave >> 1, head = 2 * g + h;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
+    const int h = wave & 1, sp = wave >> 1;
     const int col = lane & 31, hf = lane >> 5;
     const int b0 = qb * kFaRows, nrows = min(kFaRows, rows - b0);
     const int last = pos0 + b0 + nrows - 1;  // last key any query of the block attends to
@@ -207,63 +245,97 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     const int qpos = pos0 + b0 + col;        // causal limit of this lane's query
     const float scale2 = scale * 1.4426950408889634f;
 
-    // Direct loads of step i: split sp's tile kt = 4 i + sp; load j of this
-    // wave fills 16-byte slot 64 (2 j + h) + lane of the split's K tile
-    // (j < 4) or V tile; rows past `last` repeat row `last` (masked).
-    int ld_row[8], ld_col[8];
+    // Query rows 8 sp + lane / 8 of head h for the workgroup's Q^T operands, 16
+    // channels per lane (rows past the chunk repeat its last row and are
+    // never written).
+    const int q_row = 8 * sp + (lane >> 3), q_lane = lane & 7;
+    float qv[4][4];
+    {
+        const float* src = QKV + size_t(b0 + min(q_row, nrows - 1)) * kQKVRows + (2 * g + h) * kHeadDim + 4 * q_lane;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int q = (64 * (2 * j + h) + lane) & 511, r = q >> 4;
-        ld_row[j] = r;
-        ld_col[j] = 8 * ((q & 15) ^ fb_swz(r));
+        for (int i = 0; i < 4; ++i) {
+            const float4 x = *reinterpret_cast<const float4*>(src + 32 * i);
+            qv[i][0] = x.x, qv[i][1] = x.y, qv[i][2] = x.z, qv[i][3] = x.w;
+        }
     }
-    auto issue = [&](int step) {
-        const int kt = 4 * step + sp;
-        unsigned char* dst = lds + (step & 1) * kFbStageBytes + sp * kFbSplitBytes;
-        if (kt < ntiles) {
+
+    // Direct loads of step i: split sp's tile kt = 4 i + sp; load j of this
+    // wave fills 16-byte slot 64 (2 j + h) + lane of the K or V tile; rows past
+    // `last` repeat row `last` (masked).
+    int ld_row[4];
+    unsigned ld_col[4];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int key = min(kt * kFaKeys + ld_row[j], last);
-                const uint16_t* src = (j < 4 ? keys : values) + (head_base + key) * kHeadDim + ld_col[j];
-                load_lds16(src, dst + 1024 * (2 * j + h));
-            }
+    for (int j = 0; j < 4; ++j) {
+        const int q = 64 * (2 * j + h) + lane, r = q >> 4;
+        ld_row[j] = r;
+        ld_col[j] = 16 * ((q & 15) ^ fb_swz(r));
+    }
+    auto issue = [&](const uint16_t* cache, int step, int v) {
+        const int kt = 4 * step + sp;
+        const unsigned dst = lds0 + sp * kFbSplitBytes + (2 * v + (step & 1)) * kFbTileBytes + 1024 * h;
+        if (kt < ntiles) {
+            const uint16_t* first = cache + (head_base + size_t(kt) * kFaKeys) * kHeadDim;
+            const int rows_left = last - kt * kFaKeys;  // row `last` of the tile, 31 or more within
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                load_lds16_opaque(first, unsigned(min(ld_row[j], rows_left)) * (kHeadDim * 2) + ld_col[j], dst + 2048 * j);
         }
     };
-    issue(0);
+    issue(keys, 0, 0);
 
-    // Q^T operand: query b0 + col (rows past the chunk repeat its last row
-    // and are never written), channels 16s + 8hf .. +7, scaled by
-    // scale * log2(e) so that the scores come out in the exp2 domain.
-    // A query row whose largest magnitude reaches 65504 is split as
-    // q * 2^-eq (split_exponent) and its scores scaled back by 2^eq.
-    half8 qh[8], ql[8];
-    int eq;
+    // The queries, scaled by scale * log2(e) so that the scores come out in the
+    // exp2 domain, as FP16 hi / lo planes [head][plane][row] in the V buffers
+    // 1 (first used by step 1). A row whose largest magnitude reaches 65504 is
+    // split as q * 2^-e (split_exponent) and its scores scaled back by 2^e.
+    auto q_plane = [&](int head, int plane) { return lds + (2 * head + plane) * kFbSplitBytes + 3 * kFbTileBytes; };
     {
-        const float* qrow = QKV + size_t(b0 + min(col, nrows - 1)) * kQKVRows + head * kHeadDim + 8 * hf;
-        float v[8][8], big = 0.f;
+        float big = 0.f;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const float4 x0 = reinterpret_cast<const float4*>(qrow + 16 * s)[0];
-            const float4 x1 = reinterpret_cast<const float4*>(qrow + 16 * s)[1];
-            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                v[s][i] = x[i] * scale2;
-                big = fmaxf(big, fabsf(v[s][i]));
+            for (int e = 0; e < 4; ++e) {
+                qv[i][e] = fp32_fixed(qv[i][e] * scale2);
+                big = fmaxf(big, fabsf(qv[i][e]));
             }
+        const int e_row = split_exponent(max_of_8(big));
+        if (__builtin_amdgcn_ballot_w64(e_row != 0) != 0) {
+            const float down = pow2(-e_row);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) qv[i][e] = fp32_fixed(qv[i][e] * down);
         }
-        eq = split_exponent(fmaxf(big, __shfl_xor(big, 32)));
-        const float down = pow2(-eq);
+        if (q_lane == 0) q_exp[h][q_row] = e_row;
 #pragma unroll
-        for (int s = 0; s < 8; ++s)
+        for (int i = 0; i < 4; ++i) {
+            half2 hi[2], lo[2];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                _Float16 hh, ll;
-                split_half(v[s][i] * down, hh, ll);
-                qh[s][i] = hh;
-                ql[s][i] = ll;
+            for (int e = 0; e < 2; ++e) {
+                hi[e] = __builtin_convertvector(floatx2{qv[i][2 * e], qv[i][2 * e + 1]}, half2);
+                lo[e] = __builtin_convertvector(
+                    floatx2{rest_of_half<0>(hi[e], qv[i][2 * e]), rest_of_half<1>(hi[e], qv[i][2 * e + 1])}, half2);
             }
+            const int c = 4 * q_lane + 32 * i, at = 16 * fb_slot(q_row, c >> 3) + 2 * (c & 7);
+            *reinterpret_cast<half4*>(q_plane(h, 0) + at) = half4{hi[0][0], hi[0][1], hi[1][0], hi[1][1]};
+            *reinterpret_cast<half4*>(q_plane(h, 1) + at) = half4{lo[0][0], lo[0][1], lo[1][0], lo[1][1]};
+        }
     }
+    issue(values, 0, 1);
+    issue(keys, 1, 0);
+    // K tile 0 has landed: of the up to 8 later loads all may be pending.
+    if (4 + sp < ntiles) wait_vmcnt<8>();
+    else wait_vmcnt<0>();
+    wait_lgkm0();
+    stage_barrier();
+
+    // Q^T operand: query b0 + col, channels 16 s + 8 hf .. + 7.
+    half8 qh[8], ql[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        qh[s] = *reinterpret_cast<const half8*>(q_plane(h, 0) + 16 * fb_slot(col, 2 * s + hf));
+        ql[s] = *reinterpret_cast<const half8*>(q_plane(h, 1) + 16 * fb_slot(col, 2 * s + hf));
+    }
+    const int eq = q_exp[h][col];
     const bool q_scaled = __builtin_amdgcn_ballot_w64(eq != 0) != 0;
     const float q_up = pow2(eq);
     float m = -INFINITY, l = 0.f;
@@ -278,62 +350,100 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     // 32 dt + 16 (G % 2) + 4 (jj % 4) (jj = j % 16).
     const int grp = lane >> 4, jj = lane & 15;
     const int tr_row = 4 * (grp >> 1) + (jj >> 2), tr_ch = 16 * (grp & 1) + 4 * (jj & 3);
-    for (int step = 0; step < nsteps; ++step) {
-        wait_vmcnt<0>();       // this wave's loads of the step have landed
-        stage_barrier();       // everyone's have; the other buffer is free again
-        if (step + 1 < nsteps) issue(step + 1);
-        const int kt = 4 * step + sp, t0 = kt * kFaKeys;
-        if (kt >= ntiles) continue;  // wave-uniform: this split has no tile in the last step
-        const unsigned char* k_lds = lds + (step & 1) * kFbStageBytes + sp * kFbSplitBytes;
-        const unsigned char* v_lds = k_lds + kFbTileBytes;
-        floatx16 st;
+    // K operand s reads piece 2 s + hf of row col: its slot's address is k_lane
+    // with 32 s folded in by xor (tile bases are multiples of 8 KiB). V operand
+    // (j, dt, hh) likewise: 64 dt and 32 hh by xor, then 16 j + 8 hh rows on.
+    const unsigned k_lane = lds0 + sp * kFbSplitBytes + 16 * fb_slot(col, hf);
+    const unsigned v_lane = lds0 + sp * kFbSplitBytes + 2 * kFbTileBytes + 16 * fb_slot(tr_row, tr_ch >> 3) + 2 * (tr_ch & 7);
+    floatx16 st;
+    half8 vv[8], ph[2], pl[2];
+    // P^T k slot 8 hf + i of key step j is key 16 j + 8 (i / 4) + 4 hf + i % 4;
+    // transpose load hh covers keys 16 j + 8 hh + 4 hf + 0..3 of channel
+    // 32 dt + lane % 32, the same order.
+    auto multiply_v = [&](int j) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv[4 * j + dt], ph[j], acc[dt], 0, 0, 0);
+            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv[4 * j + dt], pl[j], acc[dt], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    half8 kk[8];
+    auto read_k = [&](int step, int half) {
+        const unsigned at = k_lane + (step & 1) * kFbTileBytes;
+#pragma unroll
+        for (int s = 4 * half; s < 4 * half + 4; ++s) kk[s] = lds_read16(at ^ (32 * s));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply_k = [&] {
 #pragma unroll
         for (int r = 0; r < 16; ++r) st[r] = 0.f;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const half8 ka = *reinterpret_cast<const half8*>(k_lds + 16 * fb_slot(col, 2 * s + hf));
-            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[s], st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[s], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk[s], qh[s], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk[s], ql[s], st, 0, 0, 0);
         }
+    };
+    // Vector phase of step `step`: V operands into registers, then the online
+    // softmax: register r of st holds key t0 + 8(r/4) + 4hf + r%4. A tile
+    // entirely at or before the block's first query needs no causal mask (and
+    // its maximum is finite), which saves the per-key compares and selects on
+    // all but the diagonal tiles.
+    auto vector_phase = [&](int step) {
+        const int t0 = (4 * step + sp) * kFaKeys;
+        const unsigned at = v_lane + (step & 1) * kFbTileBytes;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                const short4_t lo4 = lds_read_tr16((at ^ (64 * dt)) + 4096 * j);
+                const short4_t hi4 = lds_read_tr16((at ^ (64 * dt) ^ 32) + 4096 * j + 2048);
+                vv[4 * j + dt] = __builtin_bit_cast(half8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+        __builtin_amdgcn_sched_barrier(0);
         if (q_scaled) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) st[r] *= q_up;
         }
-        // Online softmax; register r holds key t0 + 8(r/4) + 4hf + r%4. A
-        // tile entirely at or before the block's first query needs no causal
-        // mask (and its maximum is finite), which saves the per-key compares
-        // and selects on all but the diagonal tiles.
-        float sv[16], mnew, factor, psum = 0.f;
+        float mnew, factor, psum = 0.f;
         bool grow;
-        half8 ph[2], pl[2];
         auto softmax = [&](auto masked) {
             constexpr bool kMask = decltype(masked)::value;
             float tmax = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int t = t0 + 8 * (r >> 2) + 4 * hf + (r & 3);
-                sv[r] = !kMask || t <= qpos ? st[r] : -INFINITY;
-                tmax = fmaxf(tmax, sv[r]);
+                if constexpr (kMask) st[r] = t <= qpos ? st[r] : -INFINITY;
+                tmax = fmaxf(tmax, st[r]);
             }
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+            tmax = fmaxf(tmax, lane_xor32(tmax));
             grow = tmax > m + kFaLazyMax;  // per query (both halves agree)
             mnew = grow ? tmax : m;
             factor = !grow ? 1.f : m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mnew);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float p = kMask && sv[r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sv[r] - mnew);
-                psum += p;
-                _Float16 hh, ll;
-                split_half(p, hh, ll);
-                ph[r >> 3][r & 7] = hh;
-                pl[r >> 3][r & 7] = ll;
+            for (int r = 0; r < 16; r += 2) {
+                // Both planes of two probabilities: hi rounded, lo the exact
+                // rest rounded (no product feeds the conversions).
+                float p[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    p[e] = kMask && st[r + e] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(st[r + e] - mnew);
+                psum += p[0];
+                psum += p[1];
+                const half2 hi = __builtin_convertvector(floatx2{p[0], p[1]}, half2);
+                const half2 lo = __builtin_convertvector(floatx2{rest_of_half<0>(hi, p[0]), rest_of_half<1>(hi, p[1])},
+                                                         half2);
+                ph[r >> 3][r & 7] = hi[0];
+                ph[r >> 3][(r & 7) + 1] = hi[1];
+                pl[r >> 3][r & 7] = lo[0];
+                pl[r >> 3][(r & 7) + 1] = lo[1];
             }
         };
         if (t0 + kFaKeys - 1 <= pos0 + b0)
             softmax(std::false_type{});
         else
             softmax(std::true_type{});
-        psum += __shfl_xor(psum, 32);
+        psum += lane_xor32(psum);
         l = l * factor + psum;
         // Rescaling by 1 changes nothing; skip it when no lane's reference moved.
         if (__builtin_amdgcn_ballot_w64(grow) != 0) {
@@ -343,77 +453,90 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
                 for (int r = 0; r < 16; ++r) acc[dt][r] *= factor;
         }
         m = mnew;
-        // P^T k slot 8 hf + i of key step j is key 16 j + 8 (i / 4) + 4 hf + i % 4;
-        // transpose load hh covers keys 16 j + 8 hh + 4 hf + 0..3 of channel
-        // 32 dt + lane % 32, the same order.
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                const int c = 32 * dt + tr_ch;
-                const int r0 = 16 * j + tr_row, r1 = r0 + 8;
-                const short4_t lo4 = lds_read_tr16(v_lds + 16 * fb_slot(r0, c >> 3) + 2 * (c & 7));
-                const short4_t hi4 = lds_read_tr16(v_lds + 16 * fb_slot(r1, c >> 3) + 2 * (c & 7));
-                const half8 a = __builtin_bit_cast(half8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
-                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[j], acc[dt], 0, 0, 0);
-                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[j], acc[dt], 0, 0, 0);
-            }
+    };
+    // Every wave passes 2 nsteps + 1 barriers: splits 2 and 3 start one phase
+    // later. Only the last step can lack a tile of a split.
+    const bool late = sp >= 2;
+    auto has = [&](int step) { return 4 * step + sp < ntiles; };
+    wait_lgkm0();  // the Q planes are read: V tile 1 may replace them
+    if (late) stage_barrier();
+    if (has(0)) {
+        read_k(0, 0);
+        read_k(0, 1);
+        multiply_k();
     }
+    for (int step = 0; step + 1 < nsteps; ++step) {
+        wait_vmcnt<0>();  // this wave's loads of K tile step + 1 and V tile step
+        stage_barrier();
+        // K buffer step and V buffer step - 1 have been read by both waves.
+        issue(keys, step + 2, 0);
+        issue(values, step + 1, 1);
+        vector_phase(step);
+        wait_lgkm0();
+        stage_barrier();
+        if (has(step + 1)) read_k(step + 1, 0);
+        multiply_v(0);
+        if (has(step + 1)) read_k(step + 1, 1);
+        multiply_v(1);
+        if (has(step + 1)) multiply_k();
+    }
+    wait_vmcnt<0>();
+    stage_barrier();
+    if (has(nsteps - 1)) vector_phase(nsteps - 1);
+    wait_lgkm0();
+    stage_barrier();
+    if (has(nsteps - 1)) {
+        multiply_v(0);
+        multiply_v(1);
+    }
+    if (!late) stage_barrier();
 
     // Merge the 4 splits of each head: O^T register r of tile dt is channel
     // 32dt + 8(r/4) + 4hf + r%4 of query col.
-    stage_barrier();  // every wave is done with the K/V stages (all loads were waited for)
+    // Every wave is done with the K/V buffers (the barriers above).
     float(*facc)[kFaccPitch] = reinterpret_cast<float(*)[kFaccPitch]>(lds + wave * kFaRows * kFaccPitch * 4);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) facc[col][32 * dt + 8 * (r >> 2) + 4 * hf + (r & 3)] = acc[dt][r];
+        for (int r = 0; r < 16; r += 4)
+            *reinterpret_cast<floatx4*>(&facc[col][32 * dt + 2 * r + 4 * hf]) =
+                floatx4{acc[dt][r], acc[dt][r + 1], acc[dt][r + 2], acc[dt][r + 3]};
     if (hf == 0) {
         fm[wave][col] = m;
         fl[wave][col] = l;
     }
     __syncthreads();
-    // Thread -> head hm = tid / 256, query q, channels c0 .. c0 + 15.
-    const int hm = tid >> 8, q = (tid >> 3) & 31, c0 = (tid & 7) * 16;
-    if (q < nrows) {
+    // Half wave -> one query of a head at a time, 4 channels per lane.
+    const int c0 = 4 * (tid & 31);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int hm = k >> 1, q = (tid >> 5) + 16 * (k & 1);
+        if (q >= nrows) continue;
         float mx = fm[hm][q];
 #pragma unroll
         for (int s = 1; s < 4; ++s) mx = fmaxf(mx, fm[2 * s + hm][q]);
-        float e[4], lsum = 0.f;
+        float o[4] = {0.f, 0.f, 0.f, 0.f}, lsum = 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int w = 2 * s + hm;
-            e[s] = fm[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fm[w][q] - mx);
-            lsum = __builtin_fmaf(e[s], fl[w][q], lsum);
+            const float e = fm[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fm[w][q] - mx);
+            lsum = __builtin_fmaf(e, fl[w][q], lsum);
+            const floatx4 v = *reinterpret_cast<const floatx4*>(
+                reinterpret_cast<const float*>(lds + w * kFaRows * kFaccPitch * 4) + q * kFaccPitch + c0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(e, v[i], o[i]);
+        }
+        half4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // the O GEMM's A operand as FP16 hi / lo
+            _Float16 hh, ll;
+            split_half(o[i] / lsum, hh, ll);
+            hi[i] = hh;
+            lo[i] = ll;
         }
         const size_t out = size_t(b0 + q) * kQDim + (2 * g + hm) * kHeadDim + c0;
-        half8 hi[2], lo[2];
-#pragma unroll
-        for (int k4 = 0; k4 < 4; ++k4) {
-            float o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const float4 v = *reinterpret_cast<const float4*>(
-                    reinterpret_cast<const float*>(lds + (2 * s + hm) * kFaRows * kFaccPitch * 4) + q * kFaccPitch +
-                    c0 + 4 * k4);
-                o[0] = __builtin_fmaf(e[s], v.x, o[0]);
-                o[1] = __builtin_fmaf(e[s], v.y, o[1]);
-                o[2] = __builtin_fmaf(e[s], v.z, o[2]);
-                o[3] = __builtin_fmaf(e[s], v.w, o[3]);
-            }
-#pragma unroll
-            for (int e4 = 0; e4 < 4; ++e4) {  // the O GEMM's A operand as FP16 hi / lo
-                const float v = o[e4] / lsum;
-                _Float16 hh, ll;
-                split_half(v, hh, ll);
-                hi[k4 >> 1][4 * (k4 & 1) + e4] = hh;
-                lo[k4 >> 1][4 * (k4 & 1) + e4] = ll;
-            }
-        }
-        *reinterpret_cast<half8*>(att_hi + out) = hi[0];
-        *reinterpret_cast<half8*>(att_hi + out + 8) = hi[1];
-        *reinterpret_cast<half8*>(att_lo + out) = lo[0];
-        *reinterpret_cast<half8*>(att_lo + out + 8) = lo[1];
+        *reinterpret_cast<half4*>(att_hi + out) = hi;
+        *reinterpret_cast<half4*>(att_lo + out) = lo;
     }
 }
 

@@ -40,6 +40,26 @@ __device__ __forceinline__ void load_lds16(const void* src, unsigned char* lds) 
 #endif
 }
 
+// The same load as an opaque instruction, for loops that read the LDS while
+// loads into another part of it are on their way: the compiler cannot tell
+// the parts apart and waits for every load it knows of before an LDS read.
+// base and lds (an LDS byte address) wave-uniform, offset in bytes per lane.
+// The caller waits (wait_vmcnt) before the data is read; the compiler's own
+// counted waits only become stricter by the loads it does not see.
+__device__ __forceinline__ void load_lds16_opaque(const void* base, unsigned offset, unsigned lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+                 : "memory", "m0");
+#endif
+}
+__device__ __forceinline__ unsigned lds_address(const unsigned char* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const unsigned char*)p));
+#else
+    return 0;
+#endif
+}
+
 // vmcnt <= n (expcnt and lgkmcnt unconstrained).
 template <int n>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -70,6 +90,7 @@ __device__ __forceinline__ int lane_xor32(int v) {
     return int((threadIdx.x & 32) ? r[0] : r[1]);
 }
 __device__ __forceinline__ float lane_xor16(float v) { return __int_as_float(lane_xor16(__float_as_int(v))); }
+__device__ __forceinline__ float lane_xor32(float v) { return __int_as_float(lane_xor32(__float_as_int(v))); }
 __device__ __forceinline__ double lane_xor16(double v) {
     return __hiloint2double(lane_xor16(__double2hiint(v)), lane_xor16(__double2loint(v)));
 }

@@ -326,3 +326,29 @@ def test_prefill_rows_independent_of_tile(qpkg, pack0):
             at += rows
         assert at == 700
         assert np.array_equal(m.logits().view(np.uint32), whole)
+
+
+@pytest.mark.gpu
+def test_attention_prefill_tile_counts(qpkg):
+    """Every residue of the key-tile count modulo the 4 key splits (1 to 9 tiles
+    of 32 keys, the last one whole or ragged; with 1 to 3 tiles some splits
+    have none), a diagonal inside a tile and on its edge, one to 65 queries:
+    against FP64, and bit for bit against the same queries at the end of a
+    longer call (a query's key order depends on its position alone)."""
+    rng = np.random.default_rng(91)
+    context = 300
+    keys = (0.3 * rng.standard_normal((8, context, 128))).astype(np.float16)
+    values = rng.standard_normal((8, context, 128)).astype(np.float16)
+    qkv = np.zeros((context, 4096), np.float32)
+    qkv[:, :2048] = 3 * rng.standard_normal((context, 2048)).astype(np.float32)
+    whole = qpkg.attention_prefill(qkv, keys, values, 0)
+    for end in (1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 192, 200, 255, 256, 257, 288, 300):
+        for rows in (1, 2, 31, 32, 33, 65):
+            if rows > end:
+                continue
+            pos0 = end - rows
+            got = qpkg.attention_prefill(qkv[pos0:end], keys[:, :end], values[:, :end], pos0)
+            assert np.array_equal(got.view(np.uint32), whole[pos0:end].view(np.uint32)), (pos0, rows)
+    ref = causal_attention_fp64(qkv[:, :2048].reshape(context, 16, 128), keys, values, 0)
+    err = np.abs(whole - ref)
+    assert np.all(err <= 1e-4 + 1e-4 * np.abs(ref)), float(err.max())
