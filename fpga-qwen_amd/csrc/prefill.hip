@@ -25,7 +25,6 @@ namespace qwen_hip {
 namespace {
 
 __device__ __forceinline__ float h2f(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
-__device__ __forceinline__ uint16_t f2h(float f) { return to_half_bits(f); }
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -54,7 +53,7 @@ template <int SPLITS>
 __device__ __forceinline__ float fold_splits(float x, const float* p, size_t stride) {
     static_assert(SPLITS == 0 || SPLITS == 4, "K-split GEMMs use 4 ranges");
     if constexpr (SPLITS == 0) return x;
-    else return x + ((p[0] + p[stride]) + (p[2 * stride] + p[3 * stride]));
+    else return x + (((p[0] + p[stride]) + p[2 * stride]) + p[3 * stride]);
 }
 
 
@@ -79,10 +78,10 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float* __restrict__ X
         const size_t stride = size_t(rows) * kHidden / 4;
         const float4* pr = reinterpret_cast<const float4*>(parts + size_t(b) * kHidden) + tid;
         const float4 p0 = pr[0], p1 = pr[stride], p2 = pr[2 * stride], p3 = pr[3 * stride];
-        v4.x = v4.x + ((p0.x + p1.x) + (p2.x + p3.x));
-        v4.y = v4.y + ((p0.y + p1.y) + (p2.y + p3.y));
-        v4.z = v4.z + ((p0.z + p1.z) + (p2.z + p3.z));
-        v4.w = v4.w + ((p0.w + p1.w) + (p2.w + p3.w));
+        v4.x = v4.x + (((p0.x + p1.x) + p2.x) + p3.x);
+        v4.y = v4.y + (((p0.y + p1.y) + p2.y) + p3.y);
+        v4.z = v4.z + (((p0.z + p1.z) + p2.z) + p3.z);
+        v4.w = v4.w + (((p0.w + p1.w) + p2.w) + p3.w);
         *xr = v4;
     }
     const float v[4] = {v4.x, v4.y, v4.z, v4.w};
@@ -548,33 +547,36 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(float* __restrict__ X, c
     if (idx < size_t(rows) * kHidden) X[idx] = fold_splits<SPLITS>(X[idx], parts + idx, size_t(rows) * kHidden);
 }
 
-// Tiles: rows, outputs, MFMA wave grid (outputs x rows), LDS stages, stage depth.
+// Tiles: rows, outputs, MFMA wave grid (outputs x rows), LDS stages, stage
+// depth, loaders. 8 loaders where the registers allow it and the tile is bound
+// by its loads (1-3% over 4); the smallest tiles start faster with 4.
 using Tile256 = GemmTile<128, 256, 4, 2, 2>;
 using Tile192 = GemmTile<128, 192, 2, 4, 2>;
-using Tile128 = GemmTile<128, 128, 2, 4, 3>;
-using Tile64 = GemmTile<64, 128, 4, 2, 5>;
-using Tile64n = GemmTile<64, 64, 2, 4, 6>;
+using Tile128 = GemmTile<128, 128, 2, 4, 3, 64, 8>;
+using Tile64 = GemmTile<64, 128, 4, 2, 5, 64, 8>;
+using Tile64n = GemmTile<64, 64, 2, 4, 6, 64, 8>;
 using Tile32 = GemmTile<32, 64, 2, 2, 8>;
 using Tile32n = GemmTile<32, 32, 1, 2, 6, 128>;
 using Tile16n = GemmTile<16, 32, 1, 1, 8>;
-using Qkv128 = GemmTile<128, 128, 1, 8, 3>;
-using Qkv64 = GemmTile<64, 128, 1, 4, 5>;
-using Qkv32 = GemmTile<32, 128, 1, 2, 6>;
-using Qkv16 = GemmTile<16, 128, 1, 1, 4, 128>;
+using Qkv128 = GemmTile<128, 128, 1, 8, 3, 64, 8>;
+using Qkv64 = GemmTile<64, 128, 2, 4, 5, 64, 8>;
+using Qkv32 = GemmTile<32, 128, 4, 2, 6>;
+using Qkv16 = GemmTile<16, 128, 4, 1, 4, 128, 8>;
 constexpr int kTileN = 128, kTileK = 64;  // N and K granularity of the GEMM entries
 
 template <class T, int EPI>
 void launch(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, int M, int N, int K,
             hipStream_t stream, int splits, const GemmEpilogue& ep) {
-    gemm_kernel<T, EPI><<<dim3(GemmMap(M, N, T::BM, T::BN).groups(), 1, splits), T::kThreads, 0, stream>>>(
-        Ah, Al, W, C, M, N, K, ep);
+    const GemmMap map(M, N, T::BM, T::BN, splits);
+    const GemmArgs args{Ah, Al, W, C, M, N, K, K / splits / T::TK, map.mtiles, map.ntiles, map.f, map.per, map.magic};
+    gemm_kernel<T, EPI><<<dim3(map.groups(), 1, splits), T::kThreads, 0, stream>>>(args, ep);
 }
 
 // Every CU runs one workgroup at a time, so a launch takes as many rounds as
-// it has 256 workgroups; the tile with the least rounds x price is taken. A
+// its fullest XCD has 32 workgroups; the tile with the least rounds x price is taken. A
 // price is the measured time of a round of that tile relative to 128 x 128
-// (20 us for gate/up: 16 x 32 7.0, 32 x 32 7.6, 32 x 64 8.3, 64 x 64 10.1,
-// 64 x 128 12.9, 128 x 192 28.5, 128 x 256 33; O and down within 10% of the same
+// (17.3 us for gate/up: 16 x 32 7.0, 32 x 32 7.6, 32 x 64 8.7, 64 x 64 10.3,
+// 64 x 128 12.9, 128 x 192 26, 128 x 256 30; O and down within 10% of the same
 // ratios). Tiles of short prompts keep all CUs busy: one row tile of 128 x 128
 // would leave 208 of them idle in gate/up and run 19 us.
 template <int EPI>
@@ -588,8 +590,7 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
                 const GemmEpilogue&) = nullptr;
     auto consider = [&]<class T>(double price) {
         if (N % T::BN != 0 || K % (T::TK * splits) != 0) return;
-        const long groups = long((M + T::BM - 1) / T::BM) * (N / T::BN) * splits;
-        const double cost = double((groups + 255) / 256) * price;
+        const double cost = double(GemmMap(M, N, T::BM, T::BN, splits).rounds()) * price;
         if (cost < best) {
             best = cost;
             run = &launch<T, EPI>;
@@ -607,10 +608,33 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
         consider.template operator()<Tile64n>(0.49);
         consider.template operator()<Tile64>(0.645);
         consider.template operator()<Tile128>(1.0);
-        if constexpr (EPI != kParts && EPI != kPartsGuarded) consider.template operator()<Tile192>(1.44);
-        consider.template operator()<Tile256>(1.68);
+        if constexpr (EPI != kParts && EPI != kPartsGuarded) consider.template operator()<Tile192>(1.48);
+        consider.template operator()<Tile256>(1.72);
     }
     run(Ah, Al, W, C, M, N, K, stream, splits, ep);
+}
+
+// O and down projections of `rows` rows into the residual x: 4 K ranges in
+// their own workgroups, whose partial sums the next row kernel adds, or one
+// after the other in one workgroup that adds them itself (gemm_folds). The 4
+// ranges of 128 x 128 tiles fill one round up to 1024 rows; beyond, the second
+// round and the partial sums (4 x rows x 4 KiB written and read) cost more than
+// the longer loop: O / down with the row kernel after it at 1536 rows 25.9 / 31.8
+// us in ranges, 23.1 / 29.7 folded (64 x 128 tiles), at 3072 rows 47.3 / 60.6 and
+// 33.1 / 46.8 (128 x 128 tiles); at 1024 rows 19.4 / 23.6 and 21.5 / 27.9. Whole
+// prefills of 3500 rows 12.18 -> 11.20 ms, of 3968 rows 13.47 -> 12.51.
+bool gemm_folds(int rows) { return rows > 1024; }
+
+template <bool kGuarded>
+void project_residual(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* x, float* parts, int rows, int K,
+                      hipStream_t stream, const GemmEpilogue& ep) {
+    constexpr int kRange = kGuarded ? kPartsGuarded : kParts, kWhole = kGuarded ? kFoldGuarded : kFold;
+    if (!gemm_folds(rows))
+        gemm<kRange>(Ah, Al, W, parts, rows, kHidden, K, stream, kKRanges, ep);
+    else if (GemmMap(rows, kHidden, Tile64::BM, Tile64::BN, 1).rounds() == 1)
+        launch<Tile64, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
+    else
+        launch<Tile128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
 }
 
 // FP32 rows [M x K] -> FP16 hi / lo planes (GEMM operands handed over as
@@ -746,34 +770,33 @@ void launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, con
                           hipStream_t stream) {
     require(rows >= 1 && rows <= kPrefillRows, "prefill chunk: bad row count");
     embed_rows_kernel<<<rows, 256, 0, stream>>>(ids_dev, embed, s.x);
-    // The O and down GEMMs (1024 output columns, K = 2048 / 3072) split K
-    // into 4 ranges for parallelism at any row count; the row kernel after
-    // each adds the partials to the residual in a fixed order, so a row's
-    // result still does not depend on the rows around it.
-    constexpr int kSplits = 4;
+    // Where the O and down GEMMs leave their 4 K ranges apart, the row kernel
+    // after each adds them to the residual, in the order in which the folding
+    // GEMMs do: a row's result does not depend on the rows around it.
+    const bool folded = gemm_folds(rows);
+    auto norm = [&](const float* w, bool pending, int* clear_flags) {
+        if (pending)
+            rmsnorm_rows_kernel<kKRanges><<<rows, 256, 0, stream>>>(s.x, w, s.h_hi, s.h_lo, s.part, rows, s.row_exp,
+                                                                     clear_flags);
+        else
+            rmsnorm_rows_kernel<0><<<rows, 256, 0, stream>>>(s.x, w, s.h_hi, s.h_lo, nullptr, rows, s.row_exp,
+                                                              clear_flags);
+    };
     for (int l = 0; l < kLayers; ++l) {
         const PrefillLayer& L = layers[l];
-        if (l == 0)
-            rmsnorm_rows_kernel<<<rows, 256, 0, stream>>>(s.x, L.in_norm, s.h_hi, s.h_lo, nullptr, rows, s.row_exp,
-                                                          nullptr);
-        else
-            rmsnorm_rows_kernel<kSplits><<<rows, 256, 0, stream>>>(s.x, L.in_norm, s.h_hi, s.h_lo, s.part, rows,
-                                                                   s.row_exp, nullptr);
+        norm(L.in_norm, l > 0 && !folded, nullptr);
         GemmEpilogue ep{L.q_norm, L.k_norm, cosines, sines, L.keys, L.values, pos0, context, s.act_hi, s.act_lo,
                         s.row_exp, s.act_flag, s.act_exp, false};
         gemm<kQkv>(s.h_hi, s.h_lo, L.qkv_n, s.qkv, rows, kQKVRows, kHidden, stream, 1, ep);
         launch_attention_prefill(s.qkv, L.keys, L.values, s.att_hi, s.att_lo, rows, pos0, context, stream);
         // The attention output is a convex combination of FP16 values: it fits FP16 unscaled.
-        gemm<kParts>(s.att_hi, s.att_lo, L.o_n, s.part, rows, kHidden, kQDim, stream, kSplits);
-        rmsnorm_rows_kernel<kSplits><<<rows, 256, 0, stream>>>(s.x, L.post_norm, s.h_hi, s.h_lo, s.part, rows,
-                                                               s.row_exp, s.act_flag);
+        project_residual<false>(s.att_hi, s.att_lo, L.o_n, s.x, s.part, rows, kQDim, stream, ep);
+        norm(L.post_norm, !folded, s.act_flag);
         gemm<kSwiglu>(s.h_hi, s.h_lo, L.gateup_n, nullptr, rows, 2 * kFFN, kHidden, stream, 1, ep);
-        GemmEpilogue down{};
-        down.act_flag = s.act_flag;
-        down.act_exp = s.act_exp;
-        gemm<kPartsGuarded>(s.act_hi, s.act_lo, L.down_n, s.part, rows, kHidden, kFFN, stream, kSplits, down);
+        project_residual<true>(s.act_hi, s.act_lo, L.down_n, s.x, s.part, rows, kFFN, stream, ep);
     }
-    fold_rows_kernel<kSplits><<<(rows * kHidden + 255) / 256, 256, 0, stream>>>(s.x, s.part, rows);
+    if (!folded)
+        fold_rows_kernel<kKRanges><<<(rows * kHidden + 255) / 256, 256, 0, stream>>>(s.x, s.part, rows);
 }
 
 }  // namespace qwen_hip

@@ -98,7 +98,12 @@ __device__ __forceinline__ double lane_xor32(double v) {
     return __hiloint2double(lane_xor32(__double2hiint(v)), lane_xor32(__double2loint(v)));
 }
 
-enum GemmKind { kStore, kParts, kPartsGuarded, kSwiglu, kQkv };
+// kParts: the partial products of K range blockIdx.z, stored at C + blockIdx.z
+// M N. kFold: the 4 K ranges one after the other in one workgroup, each summed
+// from zero, ((p0 + p1) + p2) + p3 added into C: the sum that the row kernels
+// form from kParts' ranges. Guarded: with the range guard of the down GEMM.
+enum GemmKind { kStore, kParts, kPartsGuarded, kFold, kFoldGuarded, kSwiglu, kQkv };
+constexpr int kKRanges = 4;
 
 // Work fused into the epilogue. QKV (kQkv): QK-norm, RoPE and the K/V cache
 // writes of engine/core.cpp:395-406. Gate/up (kSwiglu): SwiGLU, written as
@@ -138,10 +143,10 @@ struct GemmEpilogue {
 // 64 bytes of loads per clock, so a stage's loads hold up the waves that issue
 // them for about as long as the stage's MFMAs take, and waves that do both can
 // do neither during the other.
-template <int BM_, int BN_, int WN_, int WM_, int NS_, int TK_ = 64>
+template <int BM_, int BN_, int WN_, int WM_, int NS_, int TK_ = 64, int kLoaders_ = 4>
 struct GemmTile {
     static constexpr int BM = BM_, BN = BN_, WN = WN_, WM = WM_, NS = NS_, TK = TK_;
-    static constexpr int kMma = WN * WM, kLoaders = 4, kThreads = 64 * (kMma + kLoaders);
+    static constexpr int kMma = WN * WM, kLoaders = kLoaders_, kThreads = 64 * (kMma + kLoaders);
     static constexpr int TN = BN / 16 / WN, TM = BM / 16 / WM;  // 16x16 result tiles per MFMA wave
     static constexpr int SL = TK / 8;                           // 16-byte slots per operand row
     static constexpr int kSubs = TK / 32;                       // 32-column steps per stage
@@ -168,18 +173,42 @@ __device__ __forceinline__ int gemm_swz(int r) {
 // Tile order. Workgroup w runs on XCD w % 8 (round-robin dispatch). The XCDs
 // form 8 / f groups of f: group i takes the row tiles i, i + 8 / f, ... and its
 // XCDs split the column tiles by residue mod f, so each W tile is fetched by
-// 8 / f XCDs and each A row by f. Short prompts (few row tiles) are bound by
-// the weights: every W tile goes to one XCD (f = 8). With 4 or more row tiles
-// per XCD its 32 CUs share rows and columns within the L2 at f = 1.
+// 8 / f XCDs and each A row by f. Short prompts (few row tiles, bound by the
+// weights) send every W tile to one XCD (f = 8); with 4 or more row tiles per
+// XCD its 32 CUs share rows and columns within the L2 at f = 1 (gate/up of 3968
+// rows 93 us, 107 at f = 8). Another f is taken only where it saves a round: 5 row
+// tiles of 64 in gate/up at f = 4 give half of the XCDs 36 workgroups for their
+// 32 CUs, 23 us instead of 13.
 struct GemmMap {
-    int mtiles, ntiles, f, per;  // per: row tiles of a group
-    __host__ __device__ GemmMap(int M, int N, int BM, int BN) {
+    int mtiles, ntiles, splits, f, per;  // per: row tiles of a group
+    unsigned magic;                      // slot / per = (slot * magic) >> 32 (slot x per < 2^32)
+    GemmMap(int M, int N, int BM, int BN, int k_splits) {
         mtiles = (M + BM - 1) / BM;
         ntiles = N / BN;
+        splits = k_splits;
         f = mtiles <= 4 ? 8 : mtiles <= 8 ? 4 : mtiles < 25 ? 2 : 1;
-        per = (mtiles + 8 / f - 1) / (8 / f);
+        for (int g : {8, 4, 2, 1})
+            if (rounds(g) < rounds(f)) f = g;
+        per = rows(f);
+        magic = unsigned(((1ull << 32) + per - 1) / per);
     }
-    __host__ __device__ int groups() const { return 8 * per * ((ntiles + f - 1) / f); }
+    int rows(int g) const { return (mtiles + 8 / g - 1) / (8 / g); }
+    long tiles(int g) const { return long(rows(g)) * ((ntiles + g - 1) / g); }  // of the fullest XCD, per K split
+    long rounds(int g) const { return (tiles(g) * splits + 31) / 32; }
+    long rounds() const { return rounds(f); }
+    unsigned groups() const { return unsigned(8 * tiles(f)); }
+};
+
+// Launch arguments: the operands, the shape and the tile order.
+struct GemmArgs {
+    const uint16_t* Ah;
+    const uint16_t* Al;
+    const uint16_t* W;
+    float* C;
+    int M, N, K;
+    int nk;  // stages of a workgroup's K range
+    int mtiles, ntiles, f, per;
+    unsigned magic;
 };
 
 // gate * sigmoid(gate) * up with sigmoid(g) = 0.5 + 0.5 tanh(g / 2)
@@ -193,32 +222,35 @@ __device__ __forceinline__ float swiglu(float gate, float up) {
 }
 
 template <class T, int EPI>
-__global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __restrict__ Ah,
-                                                           const uint16_t* __restrict__ Al,
-                                                           const uint16_t* __restrict__ W, float* __restrict__ C, int M,
-                                                           int N, int K, GemmEpilogue ep) {
+__global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, const GemmEpilogue ep) {
+    const uint16_t *Ah = args.Ah, *Al = args.Al, *W = args.W;
+    float* C = args.C;
+    const int M = args.M, N = args.N, K = args.K, nk = args.nk;
     constexpr int BM = T::BM, BN = T::BN, WN = T::WN, TN = T::TN, TM = T::TM, NS = T::NS, TK = T::TK, SL = T::SL;
     constexpr int kLoads = T::kLoads, kStageBytes = T::kStageBytes, kPlane = T::kPlane;
-    static_assert(EPI != kQkv || (WN == 1 && BN == kHeadDim), "a wave of the QKV epilogue holds whole heads");
+    constexpr bool kIsFold = EPI == kFold || EPI == kFoldGuarded;
+    constexpr bool kGuarded = EPI == kPartsGuarded || EPI == kFoldGuarded;
+    static_assert(EPI != kQkv || (BN == kHeadDim && TN % 2 == 0), "a QKV wave holds both channels of its RoPE pairs");
     static_assert(EPI != kSwiglu || TN % 2 == 0, "a wave of the SwiGLU epilogue holds gate and up tiles");
-    // Results staged for the stores, over the ring: QKV rows of a wave, the
-    // SwiGLU planes or the C tile of the workgroup; pitches 16 bytes past a
-    // multiple of the banks.
+    // Results staged for the stores, over the ring: QKV rows (and the waves'
+    // shares of the row sums), the SwiGLU planes or the C tile of the
+    // workgroup; pitches 16 bytes past a multiple of the banks.
     constexpr int kPitch = EPI == kQkv ? 4 * kHeadDim + 16 : EPI == kSwiglu ? BN + 16 : 4 * BN + 16;  // bytes
-    constexpr int kOutBytes = EPI == kQkv ? T::kMma * 16 * kPitch : EPI == kSwiglu ? 2 * BM * kPitch : BM * kPitch;
+    constexpr int kOutBytes = EPI == kQkv ? BM * kPitch + 4 * BM * 8 : EPI == kSwiglu ? 2 * BM * kPitch : BM * kPitch;
     constexpr int kSmem = NS * kStageBytes > kOutBytes ? NS * kStageBytes : kOutBytes;
     static_assert(kSmem <= 160 * 1024, "LDS");
     __shared__ __align__(16) unsigned char smem[kSmem];
     const int tid = threadIdx.x, lane = tid & 63;
-    const GemmMap map(M, N, BM, BN);
-    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, groups = 8 / map.f;
-    const int mt = xcd / map.f + groups * (slot % map.per), nt = xcd % map.f + map.f * (slot / map.per);
-    if (mt >= map.mtiles || nt >= map.ntiles) return;
+    const unsigned xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int cc = args.per == 1 ? int(slot) : int((static_cast<unsigned long long>(slot) * args.magic) >> 32);
+    const int rr = int(slot) - cc * args.per, shift = 31 - __builtin_clz(args.f);
+    const int mt = int(xcd >> shift) + (8 >> shift) * rr, nt = int(xcd & (args.f - 1)) + args.f * cc;
+    if (mt >= args.mtiles || nt >= args.ntiles) return;
     const int m0 = mt * BM, n0 = nt * BN;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool mma = wave < T::kMma;
     const int wn = wave % WN, wm = wave / WN % T::WM;
-    const int ks = K / gridDim.z, kz = blockIdx.z * ks, nk = ks / TK;  // this workgroup's K range
+    const int kz = blockIdx.z * nk * TK;  // this workgroup's K range
     const int row = lane & 15, quad = lane >> 4;  // result row and output group of this lane
 
     // Loader i's load j fills slots 64 (i + 4 j) + lane of a stage: A hi, A lo,
@@ -268,11 +300,17 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
         }
     };
 
-    int flag0 = 0, flag1 = 0;  // range flags of the workgroup's rows, read by every wave
-    if constexpr (EPI == kPartsGuarded) {
-        flag0 = ep.act_flag[size_t(min(m0 + lane % BM, M - 1)) * 4 + blockIdx.z];
-        if constexpr (BM > 64) flag1 = ep.act_flag[size_t(min(m0 + 64 + lane, M - 1)) * 4 + blockIdx.z];
+    int flagged = 0;  // nonzero: a row of the workgroup has a range flag (every wave reads them all)
+    if constexpr (kGuarded) {
+        for (int r = lane; r < BM; r += 64) {
+            const int* flags = ep.act_flag + size_t(min(m0 + r, M - 1)) * 4;
+            if constexpr (kIsFold) flagged |= flags[0] | flags[1] | flags[2] | flags[3];
+            else flagged |= flags[blockIdx.z];
+        }
     }
+    // Stages of a K range of kFold, and the sum of the ranges so far.
+    const int range = nk / kKRanges;
+    floatx4 total[kIsFold ? TN : 1][kIsFold ? TM : 1];
 
     floatx4 acc[TN][TM];
     auto clear = [&] {
@@ -288,9 +326,11 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
         return stage + 16 * (SL * row + ((4 * sub + quad) ^ gemm_swz<TK>(row)));
     };
     // Output tile i of this wave starts at W row w_row(i) of the tile: gate
-    // tiles then their up tiles (SwiGLU), else in order.
+    // tiles then their up tiles (SwiGLU), a residue mod WN, so that tiles i and
+    // i + TN / 2 are 64 rows apart (QKV), else in order.
     auto w_row = [&](int i) {
         if constexpr (EPI == kSwiglu) return 16 * (wn * (TN / 2) + i % (TN / 2)) + (i < TN / 2 ? 0 : BN / 2);
+        if constexpr (EPI == kQkv) return 16 * (wn + WN * i);
         return 16 * (wn * TN + i);
     };
     auto read_w = [&](const unsigned char* at, int i) {
@@ -310,6 +350,26 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+
+    // kFold: range z of `range` stages is complete; its sum, scaled by `scale(t)`,
+    // joins the total.
+    auto fold_range = [&](int z, auto&& scale) {
+        if constexpr (kIsFold) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+                const float sc = scale(t);
+#pragma unroll
+                for (int i = 0; i < TN; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float p = acc[i][t][e] * sc;
+                        total[i][t][e] = z == 0 ? p : total[i][t][e] + p;
+                    }
+            }
+            clear();
+        }
+    };
+    auto one = [](int) { return 1.f; };
 
     int rexp[TM];
     if (!mma) {
@@ -333,7 +393,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
         // its first MFMAs. The barrier that hands over the next stage comes
         // between the halves of a stage's last step, when every operand of the
         // stage is in registers.
-        if constexpr (EPI != kParts && EPI != kPartsGuarded) {
+        if constexpr (EPI == kStore || EPI == kSwiglu || EPI == kQkv) {
 #pragma unroll
             for (int t = 0; t < TM; ++t) rexp[t] = ep.row_exp[min(m0 + (wm * TM + t) * 16 + row, M - 1)];
         }
@@ -347,7 +407,14 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
 #pragma unroll
             for (int t = 0; t < TM; ++t) h[t] = read_a(at, 0, t);
         }
+        int z = 0, range_end = range;
         for (int kt = 0; kt < nk; ++kt) {
+            if constexpr (kIsFold) {
+                if (kt == range_end) {
+                    fold_range(z++, one);
+                    range_end += range;
+                }
+            }
             const unsigned char* stage = smem + (kt % NS) * kStageBytes;
 #pragma unroll
             for (int sub = 0; sub < T::kSubs; ++sub) {
@@ -377,6 +444,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
             }
         }
         wait_lgkm0();
+        fold_range(z, one);
     }
 
     // Guarded down GEMM: the loop again with each A group rescaled in LDS to its
@@ -384,11 +452,17 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
     // than 1), one stage at a time. Every wave read the same flags, so every
     // wave takes the same branch.
     bool rescaled = false;
-    if constexpr (EPI == kPartsGuarded) {
-        if (__builtin_amdgcn_ballot_w64(flag0 != 0 || flag1 != 0) != 0) {
+    if constexpr (kGuarded) {
+        if (__builtin_amdgcn_ballot_w64(flagged != 0) != 0) {
             rescaled = true;
             clear();
+            auto row_flag = [&](int m, int z) { return ep.act_flag[size_t(min(m, M - 1)) * 4 + z]; };
+            auto range_scale = [&](int z) {
+                return [&, z](int t) { return pow2(row_flag(m0 + (wm * TM + t) * 16 + row, z)); };
+            };
             for (int kt = 0; kt < nk; ++kt) {
+                const int z = kIsFold ? kt / range : int(blockIdx.z);
+                if (kIsFold && mma && kt > 0 && kt % range == 0) fold_range(z - 1, range_scale(z - 1));
                 stage_barrier();  // every wave is done with the stage before (all loads were waited for)
                 unsigned char* stage = smem + (kt % NS) * kStageBytes;
                 if (!mma) {
@@ -398,7 +472,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
                 stage_barrier();
                 for (int q = tid; q < kPlane; q += T::kThreads) {
                     const int r = q / SL, p = (q % SL) ^ gemm_swz<TK>(r), m = min(m0 + r, M - 1);
-                    const int er = ep.act_flag[size_t(m) * 4 + blockIdx.z];
+                    const int er = row_flag(m, z);
                     if (er != 0) {
                         const int e8 = ep.act_exp[size_t(m) * (K / 8) + (kz + kt * TK) / 8 + p];
                         const float sc = pow2(e8 - er);
@@ -434,11 +508,12 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
                     wait_lgkm0();
                 }
             }
+            if (mma) fold_range(kKRanges - 1, range_scale(kKRanges - 1));
         }
     }
     stage_barrier();  // every wave is done with the ring: the results are staged over it
 
-    if constexpr (EPI <= kPartsGuarded) {
+    if constexpr (EPI <= kFoldGuarded) {
         if (mma) {
 #pragma unroll
             for (int t = 0; t < TM; ++t) {
@@ -451,7 +526,9 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
                 }
 #pragma unroll
                 for (int i = 0; i < TN; ++i) {
-                    floatx4 v = acc[i][t];
+                    floatx4 v;
+                    if constexpr (kIsFold) v = total[i][t];
+                    else v = acc[i][t];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] *= sc;
                     *reinterpret_cast<floatx4*>(smem + r * kPitch + 4 * (w_row(i) + 4 * quad)) = v;
@@ -465,8 +542,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
             if (m < M) {
                 floatx4 v = *reinterpret_cast<const floatx4*>(smem + r * kPitch + 16 * c4);
                 floatx4* c = reinterpret_cast<floatx4*>(C + (size_t(blockIdx.z) * M + m) * N + n0) + c4;
-                if constexpr (EPI == kStore) {
-                    if (ep.add) {
+                if constexpr (EPI == kStore || kIsFold) {
+                    if (kIsFold || ep.add) {
                         const floatx4 o = *c;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) v[e] = o[e] + v[e];
@@ -523,109 +600,140 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const uint16_t* __res
                     *reinterpret_cast<const u32x4*>(smem + rp * kPitch + 16 * c8);
             }
         }
-    } else if (mma) {
-        // Head nt of rows m: this lane holds channels j = 16 i + 4 quad + e
-        // (i < 8, e < 4), so the RoPE pair (j, j + 64) is in tiles i and i + 4.
+    } else {
+        // Head nt of rows m: this lane holds channels j = w_row(i) + 4 quad + e
+        // (i < TN, e < 4), so the RoPE pair (j, j + 64) is in tiles i and
+        // i + TN / 2.
         const int head = nt;
         const bool is_q = head < kQHeads, is_v = head >= kQHeads + kKVHeads;
-        unsigned char* out = smem + wave * 16 * kPitch;  // this wave's rows
+        // Row sums of the QK-norm (FP32 squares, FP64 sum, engine/core.cpp:
+        // 207-215) in an order that does not depend on the tile: the tiles w
+        // and w + 4 of a head together, then (0 + 1) + (2 + 3).
+        constexpr int kClasses = 4 / WN;                                 // such pairs per wave
+        double* sums = reinterpret_cast<double*>(smem + BM * kPitch);  // [4][BM]
+        double sum[TM][kClasses];
+        if (mma) {
 #pragma unroll
-        for (int t = 0; t < TM; ++t) {
-            const int mw = m0 + (wm * TM + t) * 16, m = mw + row;
-            const float sc = pow2(rexp[t]);
-            float x[8][4];
+            for (int t = 0; t < TM; ++t) {
+                const float sc = pow2(rexp[t]);
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[i][e] = acc[i][t][e] * sc;
-            if (is_v) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    half4 hv;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) hv[e] = to_half(x[i][e]);
-                    *reinterpret_cast<half4*>(out + row * kPitch + 2 * (16 * i + 4 * quad)) = hv;
-                }
-            } else {
-                double sum = 0.0;  // FP32 squares, FP64 sum (engine/core.cpp:207-215)
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < TN; ++i)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float square = x[i][e] * x[i][e];
-                        sum += static_cast<double>(square);
+                        acc[i][t][e] *= sc;
+                        const float square = acc[i][t][e] * acc[i][t][e];
+                        double& to = sum[t][i % kClasses];
+                        to = i < kClasses && e == 0 ? static_cast<double>(square) : to + static_cast<double>(square);
                     }
-                sum += lane_xor16(sum);
-                sum += lane_xor32(sum);
-                const float inv = 1.0f / __builtin_sqrtf(static_cast<float>(sum) / 128.0f + 1e-6f);
+#pragma unroll
+                for (int k = 0; k < kClasses; ++k) {
+                    sum[t][k] += lane_xor16(sum[t][k]);
+                    sum[t][k] += lane_xor32(sum[t][k]);
+                    if (WN > 1 && quad == 0) sums[(wn + WN * k) * BM + (wm * TM + t) * 16 + row] = sum[t][k];
+                }
+            }
+        }
+        if (WN > 1) __syncthreads();
+        if (mma) {
+#pragma unroll
+            for (int t = 0; t < TM; ++t) {
+                const int r = (wm * TM + t) * 16 + row, m = m0 + r;
+                unsigned char* out = smem + r * kPitch;
+                if (is_v) {
+#pragma unroll
+                    for (int i = 0; i < TN; ++i) {
+                        half4 hv;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) hv[e] = to_half(acc[i][t][e]);
+                        *reinterpret_cast<half4*>(out + 2 * (w_row(i) + 4 * quad)) = hv;
+                    }
+                    continue;
+                }
+                double c[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    if constexpr (WN > 1) c[w] = sums[w * BM + r];
+                    else c[w] = sum[t][w];
+                }
+                const float total = static_cast<float>((c[0] + c[1]) + (c[2] + c[3]));
+                const float inv = 1.0f / __builtin_sqrtf(total / 128.0f + 1e-6f);
                 const float* nw = (is_q ? ep.q_norm : ep.k_norm) + 4 * quad;
                 const size_t rope = size_t(ep.pos0 + min(m, M - 1)) * 64 + 4 * quad;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const floatx4 w0 = *reinterpret_cast<const floatx4*>(nw + 16 * i);
-                    const floatx4 w1 = *reinterpret_cast<const floatx4*>(nw + 16 * i + 64);
-                    const floatx4 cs = *reinterpret_cast<const floatx4*>(ep.cosines + rope + 16 * i);
-                    const floatx4 sn = *reinterpret_cast<const floatx4*>(ep.sines + rope + 16 * i);
+                for (int i = 0; i < TN / 2; ++i) {
+                    const floatx4 w0 = *reinterpret_cast<const floatx4*>(nw + w_row(i));
+                    const floatx4 w1 = *reinterpret_cast<const floatx4*>(nw + w_row(i) + 64);
+                    const floatx4 cs = *reinterpret_cast<const floatx4*>(ep.cosines + rope + w_row(i));
+                    const floatx4 sn = *reinterpret_cast<const floatx4*>(ep.sines + rope + w_row(i));
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const float a = (x[i][e] * inv) * w0[e], b = (x[i + 4][e] * inv) * w1[e];
-                        x[i][e] = a * cs[e] - b * sn[e];
-                        x[i + 4][e] = b * cs[e] + a * sn[e];
+                        const float a = (acc[i][t][e] * inv) * w0[e], b = (acc[i + TN / 2][t][e] * inv) * w1[e];
+                        acc[i][t][e] = a * cs[e] - b * sn[e];
+                        acc[i + TN / 2][t][e] = b * cs[e] + a * sn[e];
                     }
                 }
-                // Chain-permuted order (kperm): channel j = 8 s + c has its
-                // place in piece c + 8 (s / 8) at s % 8. This lane holds
-                // c = 4 (quad & 1) + e and s = 2 i + quad / 2, lane ^ 32 the
-                // other parity of s; trading the tiles i >= 4 of the lower half
-                // of the lanes for the tiles i < 4 of the upper half leaves lane
-                // half `up` with all 8 steps of the pieces c + 8 up.
-                const int piece = 4 * (quad & 1) + 8 * (lane >> 5);
+                if constexpr (WN == 1) {
+                    // Chain-permuted order (kperm): channel j = 8 s + c has its
+                    // place in piece c + 8 (s / 8) at s % 8. This lane holds
+                    // c = 4 (quad & 1) + e and s = 2 i + quad / 2, lane ^ 32 the
+                    // other parity of s; trading the tiles i >= 4 of the lower
+                    // half of the lanes for the tiles i < 4 of the upper half
+                    // leaves lane half `up` with all 8 steps of the pieces
+                    // c + 8 up.
+                    const int piece = 4 * (quad & 1) + 8 * (lane >> 5);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float y[8];
+                    for (int e = 0; e < 4; ++e) {
+                        float y[8];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x[i][e]),
-                                                                        __float_as_int(x[i + 4][e]), false, false);
-                        y[2 * i] = __int_as_float(int(r[0]));
-                        y[2 * i + 1] = __int_as_float(int(r[1]));
+                        for (int i = 0; i < 4; ++i) {
+                            const auto pair = __builtin_amdgcn_permlane32_swap(
+                                __float_as_int(acc[i][t][e]), __float_as_int(acc[i + 4][t][e]), false, false);
+                            y[2 * i] = __int_as_float(int(pair[0]));
+                            y[2 * i + 1] = __int_as_float(int(pair[1]));
+                        }
+                        if (is_q) {
+                            floatx4* q = reinterpret_cast<floatx4*>(out + 32 * (piece + e));
+                            q[0] = floatx4{y[0], y[1], y[2], y[3]};
+                            q[1] = floatx4{y[4], y[5], y[6], y[7]};
+                        } else {
+                            half8 hv;
+#pragma unroll
+                            for (int s = 0; s < 8; ++s) hv[s] = to_half(y[s]);
+                            *reinterpret_cast<half8*>(out + 16 * (piece + e)) = hv;
+                        }
                     }
-                    if (is_q) {
-                        floatx4* q = reinterpret_cast<floatx4*>(out + row * kPitch + 32 * (piece + e));
-                        q[0] = floatx4{y[0], y[1], y[2], y[3]};
-                        q[1] = floatx4{y[4], y[5], y[6], y[7]};
-                    } else {
-                        half8 hv;
+                } else {
 #pragma unroll
-                        for (int s = 0; s < 8; ++s) hv[s] = to_half(y[s]);
-                        *reinterpret_cast<half8*>(out + row * kPitch + 16 * (piece + e)) = hv;
-                    }
+                    for (int i = 0; i < TN; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int at = kperm(w_row(i) + 4 * quad + e);
+                            if (is_q) reinterpret_cast<float*>(out)[at] = acc[i][t][e];
+                            else reinterpret_cast<uint16_t*>(out)[at] = to_half_bits(acc[i][t][e]);
+                        }
                 }
             }
-            // The rows are this wave's own: whole rows out, 16 bytes per lane.
-            wait_lgkm0();
-            asm volatile("" ::: "memory");
-            if (is_q) {
+        }
+        __syncthreads();
+        // Whole rows out, 16 bytes per lane.
+        if (is_q) {
 #pragma unroll 4
-                for (int q = lane; q < 16 * 32; q += 64) {
-                    const int r = q >> 5, c4 = q & 31;
-                    if (mw + r < M)
-                        reinterpret_cast<floatx4*>(C + size_t(mw + r) * N + head * kHeadDim)[c4] =
-                            *reinterpret_cast<const floatx4*>(out + r * kPitch + 16 * c4);
-                }
-            } else {
-                uint16_t* cache = is_v ? ep.values + size_t(head - kQHeads - kKVHeads) * ep.context * kHeadDim
-                                       : ep.keys + size_t(head - kQHeads) * ep.context * kHeadDim;
-#pragma unroll
-                for (int q = lane; q < 16 * 16; q += 64) {
-                    const int r = q >> 4, c8 = q & 15;
-                    if (mw + r < M)
-                        reinterpret_cast<u32x4*>(cache + size_t(ep.pos0 + mw + r) * kHeadDim)[c8] =
-                            *reinterpret_cast<const u32x4*>(out + r * kPitch + 16 * c8);
-                }
+            for (int q = tid; q < BM * 32; q += T::kThreads) {
+                const int r = q >> 5, c4 = q & 31;
+                if (m0 + r < M)
+                    reinterpret_cast<floatx4*>(C + size_t(m0 + r) * N + head * kHeadDim)[c4] =
+                        *reinterpret_cast<const floatx4*>(smem + r * kPitch + 16 * c4);
             }
-            wait_lgkm0();
-            asm volatile("" ::: "memory");
+        } else {
+            uint16_t* cache = is_v ? ep.values + size_t(head - kQHeads - kKVHeads) * ep.context * kHeadDim
+                                   : ep.keys + size_t(head - kQHeads) * ep.context * kHeadDim;
+#pragma unroll 4
+            for (int q = tid; q < BM * 16; q += T::kThreads) {
+                const int r = q >> 4, c8 = q & 15;
+                if (m0 + r < M)
+                    reinterpret_cast<u32x4*>(cache + size_t(ep.pos0 + m0 + r) * kHeadDim)[c8] =
+                        *reinterpret_cast<const u32x4*>(smem + r * kPitch + 16 * c8);
+            }
         }
     }
 }

@@ -352,3 +352,40 @@ def test_attention_prefill_tile_counts(qpkg):
     ref = causal_attention_fp64(qkv[:, :2048].reshape(context, 16, 128), keys, values, 0)
     err = np.abs(whole - ref)
     assert np.all(err <= 1e-4 + 1e-4 * np.abs(ref)), float(err.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('rows', [1100, 2100])
+def test_prefill_folding_gemms(qpkg, pack0, rows):
+    """Beyond 1024 rows the O and down GEMMs add their 4 K ranges themselves
+    (64-row tiles, then 128-row tiles from 2049 rows): the bits of calls of at
+    most 1024 rows, whose ranges the row kernels add."""
+    prompt = PROMPTS['long_3968'][:rows]
+    with qpkg.Model(pack0) as m:
+        m.prefill(prompt)
+        whole = m.logits().view(np.uint32).copy()
+        m.reset()
+        for at in range(0, rows, 700):
+            m.prefill(prompt[at:at + 700])
+        assert np.array_equal(m.logits().view(np.uint32), whole)
+
+
+@pytest.mark.gpu
+def test_prefill_folding_gemms_range_guard(qpkg, tmp_path):
+    """The same with activations past FP16's range (norm gains of 32768 in 8
+    channels): the folding down GEMM rescales each K range of a flagged row by
+    that range's exponent, as the ranged one does."""
+    import test_export
+    path = test_export.write_full_checkpoint(tmp_path / 'model.safetensors', gains=test_export.LARGE_GAINS)
+    out = tmp_path / 'pack' / 'weights.bin'
+    test_export.export_pack.write_pack(path, out)
+    path.unlink()
+    prompt = PROMPTS['long_3968'][:1100]
+    with qpkg.Model(out, context=1200) as m:
+        m.prefill(prompt)
+        whole = m.logits().view(np.uint32).copy()
+        assert np.isfinite(whole.view(np.float32)).all()
+        m.reset()
+        m.prefill(prompt[:500])
+        m.prefill(prompt[500:])
+        assert np.array_equal(m.logits().view(np.uint32), whole)
