@@ -32,14 +32,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// FP32 value -> the FP16 hi / lo pair the GEMMs read (hi = fp16(v), lo = fp16(v - hi)).
-__device__ __forceinline__ void split_store(float v, uint16_t* hi, uint16_t* lo, size_t i) {
-    _Float16 h, l;
-    split_half(v, h, l);
-    hi[i] = __builtin_bit_cast(uint16_t, h);
-    lo[i] = __builtin_bit_cast(uint16_t, l);
-}
-
 // x[b] = fp32(E[ids[b]]) (engine/core.cpp:382-383).
 __global__ __launch_bounds__(256) void embed_rows_kernel(const int* __restrict__ ids, const uint16_t* __restrict__ E,
                                                          float* __restrict__ X) {
@@ -547,21 +539,32 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(float* __restrict__ X, c
     if (idx < size_t(rows) * kHidden) X[idx] = fold_splits<SPLITS>(X[idx], parts + idx, size_t(rows) * kHidden);
 }
 
-// Tiles: rows, outputs, MFMA wave grid (outputs x rows), LDS stages, stage
-// depth, loaders. 8 loaders where the registers allow it and the tile is bound
-// by its loads (1-3% over 4); the smallest tiles start faster with 4.
-using Tile256 = GemmTile<128, 256, 4, 2, 2>;
-using Tile192 = GemmTile<128, 192, 2, 4, 2>;
-using Tile128 = GemmTile<128, 128, 2, 4, 3, 64, 8>;
-using Tile64 = GemmTile<64, 128, 4, 2, 5, 64, 8>;
-using Tile64n = GemmTile<64, 64, 2, 4, 6, 64, 8>;
-using Tile32 = GemmTile<32, 64, 2, 2, 8>;
-using Tile32n = GemmTile<32, 32, 1, 2, 6, 128>;
-using Tile16n = GemmTile<16, 32, 1, 1, 8>;
-using Qkv128 = GemmTile<128, 128, 1, 8, 3, 64, 8>;
-using Qkv64 = GemmTile<64, 128, 2, 4, 5, 64, 8>;
-using Qkv32 = GemmTile<32, 128, 4, 2, 6>;
+// Tiles (by rows and outputs): MFMA wave grid (outputs x rows), LDS stages,
+// stage depth, loaders. 8 loaders where the registers allow it and the tile is
+// bound by its loads (1-3% over 4); the smallest tiles start faster with 4.
+using Tile16x32 = GemmTile<16, 32, 1, 1, 8>;
+using Tile32x32 = GemmTile<32, 32, 1, 2, 6, 128>;
+using Tile32x64 = GemmTile<32, 64, 2, 2, 8>;
+using Tile48x64 = GemmTile<48, 64, 2, 3, 7>;
+using Tile64x64 = GemmTile<64, 64, 2, 4, 6, 64, 8>;
+using Tile48x96 = GemmTile<48, 96, 3, 1, 6>;
+using Tile64x96 = GemmTile<64, 96, 3, 2, 5>;
+using Tile96x96 = GemmTile<96, 96, 3, 2, 4>;
+using Tile48x128 = GemmTile<48, 128, 4, 1, 5>;
+using Tile64x128 = GemmTile<64, 128, 4, 2, 5, 64, 8>;
+using Tile96x128 = GemmTile<96, 128, 4, 2, 4, 64, 8>;
+using Tile128x128 = GemmTile<128, 128, 2, 4, 3, 64, 8>;
+using Fold128x128 = GemmTile<128, 128, 2, 4, 3>;  // the sums of the ranges take the registers of 8 loaders
+using Tile64x192 = GemmTile<64, 192, 2, 4, 4>;
+using Tile96x192 = GemmTile<96, 192, 3, 2, 3>;
+using Tile128x192 = GemmTile<128, 192, 2, 4, 2>;
+using Tile128x256 = GemmTile<128, 256, 4, 2, 2>;
 using Qkv16 = GemmTile<16, 128, 4, 1, 4, 128, 8>;
+using Qkv32 = GemmTile<32, 128, 4, 2, 6>;
+using Qkv48 = GemmTile<48, 128, 2, 3, 5>;
+using Qkv64 = GemmTile<64, 128, 2, 4, 5, 64, 8>;
+using Qkv96 = GemmTile<96, 128, 1, 6, 4>;
+using Qkv128 = GemmTile<128, 128, 1, 8, 3, 64, 8>;
 constexpr int kTileN = 128, kTileK = 64;  // N and K granularity of the GEMM entries
 
 template <class T, int EPI>
@@ -573,12 +576,18 @@ void launch(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C,
 }
 
 // Every CU runs one workgroup at a time, so a launch takes as many rounds as
-// its fullest XCD has 32 workgroups; the tile with the least rounds x price is taken. A
-// price is the measured time of a round of that tile relative to 128 x 128
-// (17.3 us for gate/up: 16 x 32 7.0, 32 x 32 7.6, 32 x 64 8.7, 64 x 64 10.3,
-// 64 x 128 12.9, 128 x 192 26, 128 x 256 30; O and down within 10% of the same
-// ratios). Tiles of short prompts keep all CUs busy: one row tile of 128 x 128
-// would leave 208 of them idle in gate/up and run 19 us.
+// its fullest XCD has 32 workgroups; the tile with the least rounds x price is
+// taken. A price is the time of a full round of that tile, in us: of gate/up
+// (K 1024), of down (4 K ranges of 768; O, of 512, has the same order) and of QKV
+// (K 1024); a last round that leaves CUs idle is somewhat cheaper, more so for
+// the large tiles (QKV 128: 32 workgroups 14.5 us, 192 17.8 to 20, 256 21.9; gate/up
+// 64 x 64: 96 9.5, 192 10.8), as fewer CUs draw on the L2s, the memory and the
+// clock. Tiles of short prompts keep all CUs busy: one row tile of 128 x 128
+// would leave 208 of them idle in gate/up and run 19 us. Heights of 48 and 96
+// rows lie between the powers of two (whole prefill of 380 rows 2.10 -> 2.01 ms, of
+// 1300 rows 4.82 -> 4.44); not for the K ranges of O and down (700 rows: 96 x 128
+// 13.5 / 17.3 us on all CUs, 128 x 128 on 192 of them 12.1 / 16.1, and the row kernel
+// behind them 7.5 instead of 5.7).
 template <int EPI>
 void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, int M, int N, int K,
           hipStream_t stream, int splits = 1, const GemmEpilogue& ep = {}) {
@@ -590,26 +599,53 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
                 const GemmEpilogue&) = nullptr;
     auto consider = [&]<class T>(double price) {
         if (N % T::BN != 0 || K % (T::TK * splits) != 0) return;
-        const double cost = double(GemmMap(M, N, T::BM, T::BN, splits).rounds()) * price;
+        const GemmMap map(M, N, T::BM, T::BN, splits);
+        // A second round of small tiles of the K ranges writes its partial sums
+        // behind the first's: 48 x 128 tiles at 700 rows, priced 17, cost more
+        // than the 19 of one round of 128 x 128.
+        if (splits > 1 && T::BM < 128 && map.rounds() > 1) return;
+        const double fill = double(map.tiles(map.f) * splits - 32 * (map.rounds() - 1)) / 32;  // of the last round
+        const double share = T::BM * T::BN >= 96 * 128 ? 0.28 : 0.12;
+        const double cost = price * (double(map.rounds()) - share * (1 - fill * fill));
         if (cost < best) {
             best = cost;
             run = &launch<T, EPI>;
         }
     };
-    if constexpr (EPI == kQkv) {  // a head per tile; QKV rounds relative to Qkv128
-        consider.template operator()<Qkv16>(0.42);
-        consider.template operator()<Qkv32>(0.46);
-        consider.template operator()<Qkv64>(0.68);
-        consider.template operator()<Qkv128>(1.0);
+    if constexpr (EPI == kQkv) {  // a head per tile
+        consider.template operator()<Qkv16>(7.8);
+        consider.template operator()<Qkv32>(10.6);
+        consider.template operator()<Qkv48>(12.6);
+        consider.template operator()<Qkv64>(14.3);
+        consider.template operator()<Qkv96>(20.0);
+        consider.template operator()<Qkv128>(21.9);
+    } else if constexpr (EPI == kParts || EPI == kPartsGuarded) {
+        consider.template operator()<Tile16x32>(4.6);
+        consider.template operator()<Tile32x32>(5.3);
+        consider.template operator()<Tile32x64>(6.1);
+        consider.template operator()<Tile48x64>(7.3);
+        consider.template operator()<Tile64x64>(7.8);
+        consider.template operator()<Tile48x128>(9.0);
+        consider.template operator()<Tile64x128>(12.0);
+        consider.template operator()<Tile128x128>(22.0);
     } else {
-        consider.template operator()<Tile16n>(0.33);
-        consider.template operator()<Tile32n>(0.36);
-        consider.template operator()<Tile32>(0.40);
-        consider.template operator()<Tile64n>(0.49);
-        consider.template operator()<Tile64>(0.645);
-        consider.template operator()<Tile128>(1.0);
-        if constexpr (EPI != kParts && EPI != kPartsGuarded) consider.template operator()<Tile192>(1.48);
-        consider.template operator()<Tile256>(1.72);
+        consider.template operator()<Tile16x32>(6.6);
+        consider.template operator()<Tile32x32>(7.7);
+        consider.template operator()<Tile32x64>(8.9);
+        consider.template operator()<Tile48x64>(10.3);
+        consider.template operator()<Tile64x64>(10.8);
+        if constexpr (EPI == kSwiglu) {
+            consider.template operator()<Tile48x96>(11.9);
+            consider.template operator()<Tile64x96>(13.2);
+            consider.template operator()<Tile96x96>(16.3);
+            consider.template operator()<Tile64x192>(18.5);
+            consider.template operator()<Tile96x192>(25.8);
+            consider.template operator()<Tile128x192>(29.2);
+        }
+        consider.template operator()<Tile64x128>(14.4);
+        consider.template operator()<Tile96x128>(17.4);
+        consider.template operator()<Tile128x128>(20.3);
+        consider.template operator()<Tile128x256>(34.5);
     }
     run(Ah, Al, W, C, M, N, K, stream, splits, ep);
 }
@@ -620,8 +656,9 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
 // ranges of 128 x 128 tiles fill one round up to 1024 rows; beyond, the second
 // round and the partial sums (4 x rows x 4 KiB written and read) cost more than
 // the longer loop: O / down with the row kernel after it at 1536 rows 25.9 / 31.8
-// us in ranges, 23.1 / 29.7 folded (64 x 128 tiles), at 3072 rows 47.3 / 60.6 and
-// 33.1 / 46.8 (128 x 128 tiles); at 1024 rows 19.4 / 23.6 and 21.5 / 27.9. Whole
+// us in ranges, 23.1 / 29.7 folded (64 x 128 tiles, one round up to 2048 rows), at
+// 3072 rows 47.3 / 60.6 and 33.1 / 46.8 (128 x 128 tiles; 96 x 128 take 27.6 where
+// those take 33.6); at 1024 rows 19.4 / 23.6 and 21.5 / 27.9. Whole
 // prefills of 3500 rows 12.18 -> 11.20 ms, of 3968 rows 13.47 -> 12.51.
 bool gemm_folds(int rows) { return rows > 1024; }
 
@@ -631,21 +668,33 @@ void project_residual(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W,
     constexpr int kRange = kGuarded ? kPartsGuarded : kParts, kWhole = kGuarded ? kFoldGuarded : kFold;
     if (!gemm_folds(rows))
         gemm<kRange>(Ah, Al, W, parts, rows, kHidden, K, stream, kKRanges, ep);
-    else if (GemmMap(rows, kHidden, Tile64::BM, Tile64::BN, 1).rounds() == 1)
-        launch<Tile64, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
+    else if (GemmMap(rows, kHidden, 64, 128, 1).rounds() == 1)
+        launch<Tile64x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
+    else if (GemmMap(rows, kHidden, 96, 128, 1).rounds() == 1)
+        launch<Tile96x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
     else
-        launch<Tile128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
+        launch<Fold128x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
 }
 
 // FP32 rows [M x K] -> FP16 hi / lo planes (GEMM operands handed over as
 // FP32), one workgroup per row: the row is split as a * 2^-row_exp[m]
-// (split_exponent of its largest magnitude).
+// (split_exponent of its largest magnitude). K is a multiple of 64; rows of up to
+// 4096 columns stay in registers between the maximum and the split (341 x 3072: 5.4
+// -> 3.6 us), longer ones are read twice.
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, uint16_t* __restrict__ hi,
                                                          uint16_t* __restrict__ lo, int* __restrict__ row_exp, int K) {
+    constexpr int kHeld = 4;  // 4-column pieces per thread
     const size_t base = size_t(blockIdx.x) * K;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, pieces = K / 4;
+    const floatx4* row = reinterpret_cast<const floatx4*>(A + base);
+    floatx4 held[kHeld];
     float big = 0.f;
-    for (int i = tid; i < K; i += 256) big = fmaxf(big, fabsf(A[base + i]));
+    auto grow = [&](floatx4 v) { big = fmaxf(fmaxf(big, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3]))); };
+#pragma unroll
+    for (int k = 0; k < kHeld; ++k) held[k] = tid + 256 * k < pieces ? row[tid + 256 * k] : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kHeld; ++k) grow(held[k]);
+    for (int i = tid + 256 * kHeld; i < pieces; i += 256) grow(row[i]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off));
     __shared__ float bred[4];
@@ -654,7 +703,22 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
     const int e = split_exponent(fmaxf(fmaxf(bred[0], bred[1]), fmaxf(bred[2], bred[3])));
     const float down = pow2(-e);
     if (tid == 0) row_exp[blockIdx.x] = e;
-    for (int i = tid; i < K; i += 256) split_store(A[base + i] * down, hi, lo, base + i);
+    auto split = [&](floatx4 v, int i) {
+        half4 h4, l4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            _Float16 h, l;
+            split_half(v[k] * down, h, l);
+            h4[k] = h;
+            l4[k] = l;
+        }
+        reinterpret_cast<half4*>(hi + base)[i] = h4;
+        reinterpret_cast<half4*>(lo + base)[i] = l4;
+    };
+#pragma unroll
+    for (int k = 0; k < kHeld; ++k)
+        if (tid + 256 * k < pieces) split(held[k], tid + 256 * k);
+    for (int i = tid + 256 * kHeld; i < pieces; i += 256) split(row[i], i);
 }
 
 }  // namespace
