@@ -531,19 +531,18 @@ void Engine::run_append(const int* ids, size_t count) {
         std::copy(ids, ids + batched, ids_host_);
         HIP_CHECK(hipMemcpyAsync(ids_dev_, ids_host_, batched * sizeof(int), hipMemcpyHostToDevice, stream_));
         const int rows = int(batched);
-        launch_prefill_chunk(prefill_layers_.data(), embed_, ids_dev_, rows, pos_, cosines_, sines_,
-                             options_.context, prefill_, stream_);
+        float* final_row = launch_prefill_chunk(prefill_layers_.data(), embed_, ids_dev_, rows, pos_, cosines_, sines_,
+                                                options_.context, prefill_, stream_);
         pos_ += rows;
         if (batched == count) {
-            HIP_CHECK(hipMemcpyAsync(scratch_.x, prefill_.x + size_t(rows - 1) * kHidden, kHidden * sizeof(float),
-                                     hipMemcpyDeviceToDevice, stream_));
-            launch_lm_head(lm_t_, final_norm_, scratch_, result_host_, next_tag(), stream_);
+            DecodeScratch head = scratch_;
+            head.x = final_row;
+            launch_lm_head(lm_t_, final_norm_, head, result_host_, next_tag(), stream_, ++result_seq_);
         }
     }
     if (batched < count) run_token(ids[count - 1], true, 0);
     HIP_CHECK(hipGetLastError());
-    if (batched == 0) await_result(0);  // one row: its argmax is the call's last kernel
-    else sync();
+    await_result(0);  // the head's selection is the call's last store
     check_stall(0);
     has_logits_ = true;
 }
