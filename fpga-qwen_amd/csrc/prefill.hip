@@ -135,8 +135,8 @@ constexpr int kFaRows = 32, kFaKeys = 32, kFaccPitch = 132;
 // most tiles need no rescaling of the output accumulators.
 constexpr float kFaLazyMax = 8.f;
 
-// Workgroup = 32 consecutive query rows x one KV head g, 8 waves: wave
-// (h, s) = (wave & 1, wave >> 1) runs query head 2g + h over the key tiles
+// Workgroup = 32 consecutive query rows x one KV head g, 8 waves (HEADS = 2):
+// wave (h, s) = (wave % 2, wave / 2) runs query head 2g + h over the key tiles
 // kt = s (mod 4) with its own online softmax, and the 4 key splits of each
 // head are merged at the end. The two waves of a split load its K and V tiles
 // together (direct global -> LDS loads, two buffers of each).
@@ -210,23 +210,30 @@ __device__ __forceinline__ float max_of_8(float v) {
     return fmaxf(v, dpp(v, std::integral_constant<int, 0x141>{}));  // the other quad of 8 lanes
 }
 
-__global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __restrict__ QKV,
+// HEADS = 1: a workgroup of 4 waves runs one of the KV head's two query heads
+// (both read its K/V tiles), for few query blocks and keys: each wave has a SIMD
+// and its split's tiles to itself, so the steps need no barriers.
+template <int HEADS>
+__global__ __launch_bounds__(256 * HEADS) void attn_prefill_mfma_kernel(const float* __restrict__ QKV,
                                                                   const uint16_t* __restrict__ keys,
                                                                   const uint16_t* __restrict__ values,
                                                                   uint16_t* __restrict__ att_hi,
                                                                   uint16_t* __restrict__ att_lo, int rows, int pos0,
                                                                   int context, float scale) {
     __shared__ __align__(16) unsigned char lds[kFbLds];
-    __shared__ float fm[8][kFaRows], fl[8][kFaRows];
-    __shared__ int q_exp[2][kFaRows];
+    __shared__ float fm[4 * HEADS][kFaRows], fl[4 * HEADS][kFaRows];
+    __shared__ int q_exp[HEADS][kFaRows];
     // Workgroup w runs on XCD w % 8 (round-robin dispatch): KV head g = w % 8
     // keeps every workgroup reading one head's K/V rows on one XCD, so they
     // stay in its L2; the query blocks run heaviest (latest) first.
-    const int nqb = gridDim.x / kKVHeads;
-    const int g = blockIdx.x % kKVHeads, qb = nqb - 1 - blockIdx.x / kKVHeads;
+    constexpr int kGroups = 2 / HEADS;  // workgroups of a KV head and query block
+    const int nqb = gridDim.x / (kKVHeads * kGroups);
+    const int g = blockIdx.x % kKVHeads, block = blockIdx.x / kKVHeads;
+    const int qb = nqb - 1 - block / kGroups, first_head = 2 * g + block % kGroups;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
-    const int h = wave & 1, sp = wave >> 1;
+    const int h = wave % HEADS, sp = wave / HEADS;
+    auto phase_barrier = [] { if constexpr (HEADS == 2) stage_barrier(); };
     const int col = lane & 31, hf = lane >> 5;
     const int b0 = qb * kFaRows, nrows = min(kFaRows, rows - b0);
     const int last = pos0 + b0 + nrows - 1;  // last key any query of the block attends to
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     const int q_row = 8 * sp + (lane >> 3), q_lane = lane & 7;
     float qv[4][4];
     {
-        const float* src = QKV + size_t(b0 + min(q_row, nrows - 1)) * kQKVRows + (2 * g + h) * kHeadDim + 4 * q_lane;
+        const float* src = QKV + size_t(b0 + min(q_row, nrows - 1)) * kQKVRows + (first_head + h) * kHeadDim + 4 * q_lane;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float4 x = *reinterpret_cast<const float4*>(src + 32 * i);
@@ -251,13 +258,14 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     }
 
     // Direct loads of step i: split sp's tile kt = 4 i + sp; load j of this
-    // wave fills 16-byte slot 64 (2 j + h) + lane of the K or V tile; rows past
+    // wave fills 16-byte slot 64 (HEADS j + h) + lane of the K or V tile; rows past
     // `last` repeat row `last` (masked).
-    int ld_row[4];
-    unsigned ld_col[4];
+    constexpr int kTileLoads = 8 / HEADS;
+    int ld_row[kTileLoads];
+    unsigned ld_col[kTileLoads];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int q = 64 * (2 * j + h) + lane, r = q >> 4;
+    for (int j = 0; j < kTileLoads; ++j) {
+        const int q = 64 * (HEADS * j + h) + lane, r = q >> 4;
         ld_row[j] = r;
         ld_col[j] = 16 * ((q & 15) ^ fb_swz(r));
     }
@@ -268,8 +276,9 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
             const uint16_t* first = cache + (head_base + size_t(kt) * kFaKeys) * kHeadDim;
             const int rows_left = last - kt * kFaKeys;  // row `last` of the tile, 31 or more within
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                load_lds16_opaque(first, unsigned(min(ld_row[j], rows_left)) * (kHeadDim * 2) + ld_col[j], dst + 2048 * j);
+            for (int j = 0; j < kTileLoads; ++j)
+                load_lds16_opaque(first, unsigned(min(ld_row[j], rows_left)) * (kHeadDim * 2) + ld_col[j],
+                                  dst + 1024 * HEADS * j);
         }
     };
     issue(keys, 0, 0);
@@ -313,8 +322,8 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     }
     issue(values, 0, 1);
     issue(keys, 1, 0);
-    // K tile 0 has landed: of the up to 8 later loads all may be pending.
-    if (4 + sp < ntiles) wait_vmcnt<8>();
+    // K tile 0 has landed: of V tile 0's and K tile 1's loads all may be pending.
+    if (4 + sp < ntiles) wait_vmcnt<2 * kTileLoads>();
     else wait_vmcnt<0>();
     wait_lgkm0();
     stage_barrier();
@@ -445,42 +454,67 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
         }
         m = mnew;
     };
-    // Every wave passes 2 nsteps + 1 barriers: splits 2 and 3 start one phase
-    // later. Only the last step can lack a tile of a split.
-    const bool late = sp >= 2;
+    // HEADS = 2: every wave passes 2 nsteps + 1 barriers: splits 2 and 3 start one
+    // phase later. Only the last step can lack a tile of a split.
+    const bool late = HEADS == 2 && sp >= 2;
     auto has = [&](int step) { return 4 * step + sp < ntiles; };
     wait_lgkm0();  // the Q planes are read: V tile 1 may replace them
-    if (late) stage_barrier();
+    if (HEADS == 1 || late) stage_barrier();
     if (has(0)) {
         read_k(0, 0);
         read_k(0, 1);
         multiply_k();
     }
-    for (int step = 0; step + 1 < nsteps; ++step) {
-        wait_vmcnt<0>();  // this wave's loads of K tile step + 1 and V tile step
-        stage_barrier();
-        // K buffer step and V buffer step - 1 have been read by both waves.
-        issue(keys, step + 2, 0);
-        issue(values, step + 1, 1);
-        vector_phase(step);
-        wait_lgkm0();
-        stage_barrier();
-        if (has(step + 1)) read_k(step + 1, 0);
-        multiply_v(0);
-        if (has(step + 1)) read_k(step + 1, 1);
-        multiply_v(1);
-        if (has(step + 1)) multiply_k();
+    if constexpr (HEADS == 1) {
+        // Loads go out in two halves, V before the vector phase and K among
+        // the MFMAs: all at once, 64 KiB of them per CU stalled the 4 waves
+        // together.
+        for (int step = 0; step + 1 < nsteps; ++step) {
+            const bool next = has(step + 1);
+            // V tile step has landed; K tile step + 1 may be pending.
+            if (next) wait_vmcnt<kTileLoads>();
+            else wait_vmcnt<0>();
+            wait_lgkm0();  // V buffer step - 1 has been read
+            issue(values, step + 1, 1);
+            vector_phase(step);
+            // K tile step + 1 has landed; V tile step + 1 may be pending.
+            if (next) wait_vmcnt<kTileLoads>();
+            else wait_vmcnt<0>();
+            if (next) read_k(step + 1, 0);
+            multiply_v(0);
+            wait_lgkm0();  // K buffer step was read before
+            issue(keys, step + 2, 0);
+            if (next) read_k(step + 1, 1);
+            multiply_v(1);
+            if (next) multiply_k();
+        }
+    } else {
+        for (int step = 0; step + 1 < nsteps; ++step) {
+            wait_vmcnt<0>();  // this wave's loads of K tile step + 1 and V tile step
+            phase_barrier();
+            // K buffer step and V buffer step - 1 have been read by both waves.
+            issue(keys, step + 2, 0);
+            issue(values, step + 1, 1);
+            vector_phase(step);
+            wait_lgkm0();
+            phase_barrier();
+            if (has(step + 1)) read_k(step + 1, 0);
+            multiply_v(0);
+            if (has(step + 1)) read_k(step + 1, 1);
+            multiply_v(1);
+            if (has(step + 1)) multiply_k();
+        }
     }
     wait_vmcnt<0>();
-    stage_barrier();
+    phase_barrier();
     if (has(nsteps - 1)) vector_phase(nsteps - 1);
     wait_lgkm0();
-    stage_barrier();
+    phase_barrier();
     if (has(nsteps - 1)) {
         multiply_v(0);
         multiply_v(1);
     }
-    if (!late) stage_barrier();
+    if (HEADS == 1 || !late) stage_barrier();
 
     // Merge the 4 splits of each head: O^T register r of tile dt is channel
     // 32dt + 8(r/4) + 4hf + r%4 of query col.
@@ -501,15 +535,15 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
     const int c0 = 4 * (tid & 31);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const int hm = k >> 1, q = (tid >> 5) + 16 * (k & 1);
+        const int at = (tid >> 5) + 8 * HEADS * k, hm = at / kFaRows, q = at % kFaRows;
         if (q >= nrows) continue;
         float mx = fm[hm][q];
 #pragma unroll
-        for (int s = 1; s < 4; ++s) mx = fmaxf(mx, fm[2 * s + hm][q]);
+        for (int s = 1; s < 4; ++s) mx = fmaxf(mx, fm[HEADS * s + hm][q]);
         float o[4] = {0.f, 0.f, 0.f, 0.f}, lsum = 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int w = 2 * s + hm;
+            const int w = HEADS * s + hm;
             const float e = fm[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fm[w][q] - mx);
             lsum = __builtin_fmaf(e, fl[w][q], lsum);
             const floatx4 v = *reinterpret_cast<const floatx4*>(
@@ -525,7 +559,7 @@ __global__ __launch_bounds__(512) void attn_prefill_mfma_kernel(const float* __r
             hi[i] = hh;
             lo[i] = ll;
         }
-        const size_t out = size_t(b0 + q) * kQDim + (2 * g + hm) * kHeadDim + c0;
+        const size_t out = size_t(b0 + q) * kQDim + (first_head + hm) * kHeadDim + c0;
         *reinterpret_cast<half4*>(att_hi + out) = hi;
         *reinterpret_cast<half4*>(att_lo + out) = lo;
     }
@@ -825,8 +859,19 @@ void launch_attention_prefill(const float* qkv, const uint16_t* keys, const uint
                               uint16_t* att_lo, int rows, int pos0, int context, hipStream_t stream) {
     require(rows >= 1 && rows <= kPrefillRows && pos0 >= 0 && context > 0 && pos0 + rows <= context,
             "attention: bad rows / position / context");
-    attn_prefill_mfma_kernel<<<(rows + kFaRows - 1) / kFaRows * kKVHeads, 512, 0, stream>>>(
-        qkv, keys, values, att_hi, att_lo, rows, pos0, context, 1.0f / std::sqrt(128.0f));
+    const float scale = 1.0f / std::sqrt(128.0f);
+    const int blocks = (rows + kFaRows - 1) / kFaRows * kKVHeads;
+    // One head per workgroup while all fit one round of the 256 CUs, up to 1024
+    // keys: the start and the merge halve, but a step, its vector phase no longer
+    // beside another wave's MFMAs, takes longer. Whole prefills, two heads -> one:
+    // 85 rows 1.357 -> 1.339 ms, 17 rows behind 612 1.359 -> 1.346, behind 1000
+    // 1.463 -> 1.456, behind 1300 1.547 -> 1.564, 400 behind 3500 3.19 -> 3.28.
+    if (2 * blocks <= 256 && pos0 + rows <= 1024)
+        attn_prefill_mfma_kernel<1><<<2 * blocks, 256, 0, stream>>>(qkv, keys, values, att_hi, att_lo, rows, pos0,
+                                                                     context, scale);
+    else
+        attn_prefill_mfma_kernel<2><<<blocks, 512, 0, stream>>>(qkv, keys, values, att_hi, att_lo, rows, pos0, context,
+                                                                 scale);
 }
 
 float* launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, const int* ids_dev, int rows, int pos0,

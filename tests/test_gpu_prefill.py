@@ -355,6 +355,23 @@ def test_attention_prefill_tile_counts(qpkg):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('rows,end', [(rows, end) for rows in (1, 32, 481, 512, 513)
+                                      for end in (1, 33, 97, 512, 1024, 1025) if rows <= end])
+def test_attention_prefill_head_split(qpkg, rows, end):
+    """Up to 16 query blocks and 1024 keys a workgroup runs one query head,
+    beyond that both heads of a KV head: bit for bit the same rows out of a
+    call of 1100 rows (a head's key order and arithmetic do not depend on it)."""
+    rng = np.random.default_rng(92)
+    keys = (0.3 * rng.standard_normal((8, 1100, 128))).astype(np.float16)
+    values = rng.standard_normal((8, 1100, 128)).astype(np.float16)
+    qkv = np.zeros((1100, 4096), np.float32)
+    qkv[:, :2048] = 3 * rng.standard_normal((1100, 2048)).astype(np.float32)
+    whole = qpkg.attention_prefill(qkv, keys, values, 0)
+    got = qpkg.attention_prefill(qkv[end - rows:end], keys[:, :end], values[:, :end], end - rows)
+    assert np.array_equal(got.view(np.uint32), whole[end - rows:end].view(np.uint32))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('rows', [1100, 2100])
 def test_prefill_folding_gemms(qpkg, pack0, rows):
     """Beyond 1024 rows the O and down GEMMs add their 4 K ranges themselves
