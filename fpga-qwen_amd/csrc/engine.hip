@@ -365,8 +365,8 @@ void Engine::settle() {
     if (unsynced_) sync();
 }
 
-// A decode step returns as soon as its argmax kernel has stored the result
-// word of this launch in pinned memory (the last store of the step's last
+// A step or prefill returns as soon as its argmax kernel has stored the result
+// word of this launch in pinned memory (the last store of the call's last
 // kernel), instead of waiting for the stream's completion signal. Bounded:
 // after ~20 ms it waits for the stream, which also reports a failed launch.
 void Engine::await_result(int slot) {
