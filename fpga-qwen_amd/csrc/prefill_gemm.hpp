@@ -257,7 +257,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
     // then W rows; 64 / SL rows each. A rows past M repeat row M - 1 and are
     // never stored.
     const char* base[kLoads];   // wave-uniform
-    unsigned offset[kLoads];
+    size_t offset[kLoads];      // 64 bits: the rows of a tile may lie more than 4 GiB apart
     auto load_addresses = [&] {
         const int loader = wave - T::kMma;
 #pragma unroll
@@ -270,10 +270,10 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
                 const int r0 = r - lane / SL;
                 const int first = EPI == kSwiglu ? (r0 < BN / 2 ? n0 / 2 : N / 2 + n0 / 2 - BN / 2) : n0;
                 base[j] = reinterpret_cast<const char*>(W + size_t(first) * K + kz);
-                offset[j] = 2u * (unsigned(r) * unsigned(K) + 8u * p);
+                offset[j] = 2 * (size_t(r) * K + 8 * p);
             } else {
                 base[j] = reinterpret_cast<const char*>((q0 >= kPlane ? Al : Ah) + size_t(m0) * K + kz);
-                offset[j] = 2u * (unsigned(min(r, M - 1 - m0)) * unsigned(K) + 8u * p);
+                offset[j] = 2 * (size_t(min(r, M - 1 - m0)) * K + 8 * p);
             }
         }
     };
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
         unsigned char* stage = smem + (kt % NS) * kStageBytes + 1024 * (wave - T::kMma);
 #pragma unroll
         for (int j = 0; j < kLoads; ++j)
-            load_lds16(base[j] + offset[j] + kt * TK * 2, stage + 1024 * T::kLoaders * j);
+            load_lds16(base[j] + offset[j] + size_t(kt) * (2 * TK), stage + 1024 * T::kLoaders * j);
     };
     // Waits until at most `later` whole stages of this loader's are pending.
     auto wait_stages = [&](int later) {

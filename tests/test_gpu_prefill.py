@@ -406,3 +406,25 @@ def test_prefill_folding_gemms_range_guard(qpkg, tmp_path):
         m.prefill(prompt[:500])
         m.prefill(prompt[500:])
         assert np.array_equal(m.logits().view(np.uint32), whole)
+
+
+@pytest.mark.gpu
+def test_gemm_rows_far_apart(qpkg):
+    """W rows of 70 million halves: rows 31, 63, 95 and 127 of W begin 4.34 GB
+    behind the first row of their tile, past a 32-bit byte offset. Row n holds
+    n + 1 in column K - 1 - n alone and A ones in the last 128 columns, so the
+    products are 1 .. 128 exactly."""
+    n, k = 128, 70_000_000 // 64 * 64
+    a = np.zeros((1, k), np.float32)
+    a[0, -n:] = 1
+    ad, wd, cd = qpkg.DeviceBuffer.from_array(a), qpkg.DeviceBuffer(n * k * 2), qpkg.DeviceBuffer(n * 4)
+    lib, base = qpkg.load_library(), wd.ptr.value
+    zeros = np.zeros(1 << 28, np.uint8)
+    for at in range(0, n * k * 2, zeros.size):
+        qpkg._check(lib.qwen_gpu_memcpy_to_device(base + at, zeros.ctypes.data, min(zeros.size, n * k * 2 - at)))
+    for row in range(n):
+        value = np.full(1, row + 1, np.float16)
+        qpkg._check(lib.qwen_gpu_memcpy_to_device(base + 2 * (row * k + k - 1 - row), value.ctypes.data, 2))
+    qpkg._check(lib.qwen_gpu_op_gemm(ad.ptr, wd.ptr, cd.ptr, 1, n, k, 0, None))
+    qpkg.synchronize()
+    assert np.array_equal(cd.to_array(np.float32, n), np.arange(1, n + 1, dtype=np.float32))
