@@ -19,6 +19,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "gemm_map.hpp"
 #include "half_split.hpp"
 #include "kernels.hpp"
 #include "prefill.hpp"
@@ -170,35 +171,6 @@ __device__ __forceinline__ int gemm_swz(int r) {
     return TK == 64 ? ((r >> 1) ^ ((r & 1) << 2)) & 7 : r & 15;
 }
 
-// Tile order. Workgroup w runs on XCD w % 8 (round-robin dispatch). The XCDs
-// form 8 / f groups of f: group i takes the row tiles i, i + 8 / f, ... and its
-// XCDs split the column tiles by residue mod f, so each W tile is fetched by
-// 8 / f XCDs and each A row by f. Short prompts (few row tiles, bound by the
-// weights) send every W tile to one XCD (f = 8); with 4 or more row tiles per
-// XCD its 32 CUs share rows and columns within the L2 at f = 1 (gate/up of 3968
-// rows 93 us, 107 at f = 8). Another f is taken only where it saves a round: 5 row
-// tiles of 64 in gate/up at f = 4 give half of the XCDs 36 workgroups for their
-// 32 CUs, 23 us instead of 13.
-struct GemmMap {
-    int mtiles, ntiles, splits, f, per;  // per: row tiles of a group
-    unsigned magic;                      // slot / per = (slot * magic) >> 32 (slot x per < 2^32)
-    GemmMap(int M, int N, int BM, int BN, int k_splits) {
-        mtiles = (M + BM - 1) / BM;
-        ntiles = N / BN;
-        splits = k_splits;
-        f = mtiles <= 4 ? 8 : mtiles <= 8 ? 4 : mtiles < 25 ? 2 : 1;
-        for (int g : {8, 4, 2, 1})
-            if (rounds(g) < rounds(f)) f = g;
-        per = rows(f);
-        magic = unsigned(((1ull << 32) + per - 1) / per);
-    }
-    int rows(int g) const { return (mtiles + 8 / g - 1) / (8 / g); }
-    long tiles(int g) const { return long(rows(g)) * ((ntiles + g - 1) / g); }  // of the fullest XCD, per K split
-    long rounds(int g) const { return (tiles(g) * splits + 31) / 32; }
-    long rounds() const { return rounds(f); }
-    unsigned groups() const { return unsigned(8 * tiles(f)); }
-};
-
 // Launch arguments: the operands, the shape and the tile order.
 struct GemmArgs {
     const uint16_t* Ah;
@@ -241,10 +213,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
     static_assert(kSmem <= 160 * 1024, "LDS");
     __shared__ __align__(16) unsigned char smem[kSmem];
     const int tid = threadIdx.x, lane = tid & 63;
-    const unsigned xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int cc = args.per == 1 ? int(slot) : int((static_cast<unsigned long long>(slot) * args.magic) >> 32);
-    const int rr = int(slot) - cc * args.per, shift = 31 - __builtin_clz(args.f);
-    const int mt = int(xcd >> shift) + (8 >> shift) * rr, nt = int(xcd & (args.f - 1)) + args.f * cc;
+    const auto [mt, nt] = map_tile(blockIdx.x, args.f, args.per, args.magic);
     if (mt >= args.mtiles || nt >= args.ntiles) return;
     const int m0 = mt * BM, n0 = nt * BN;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
