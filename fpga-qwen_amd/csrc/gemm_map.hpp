@@ -4,13 +4,6 @@
 
 namespace qwen_hip {
 
-// slot / per, with magic = 2^32 / per rounded up (per > 1). The product's upper
-// half is the quotient or, where slot x per passes 2^32, at most one more.
-constexpr unsigned map_divide(unsigned slot, unsigned per, unsigned magic) {
-    const unsigned q = unsigned((static_cast<unsigned long long>(slot) * magic) >> 32);
-    return static_cast<unsigned long long>(q) * per > slot ? q - 1 : q;
-}
-
 // Tile order. Workgroup w runs on XCD w % 8 (round-robin dispatch). The XCDs
 // form 8 / f groups of f: group i takes the row tiles i, i + 8 / f, ... and its
 // XCDs split the column tiles by residue mod f, so each W tile is fetched by
@@ -22,7 +15,7 @@ constexpr unsigned map_divide(unsigned slot, unsigned per, unsigned magic) {
 // 32 CUs, 23 us instead of 13.
 struct GemmMap {
     int mtiles, ntiles, splits, f, per;  // per: row tiles of a group
-    unsigned magic;                      // 2^32 / per rounded up (map_divide)
+    unsigned magic;                      // 2^32 / per rounded up (per > 1)
     GemmMap(int M, int N, int BM, int BN, int k_splits) {
         mtiles = (M + BM - 1) / BM;
         ntiles = N / BN;
@@ -47,8 +40,15 @@ struct MapTile {
 };
 constexpr MapTile map_tile(unsigned w, int f, int per, unsigned magic) {
     const unsigned xcd = w % 8, slot = w / 8;
-    const int cc = per == 1 ? int(slot) : int(map_divide(slot, unsigned(per), magic));
-    const int rr = int(slot) - cc * per, shift = 31 - __builtin_clz(unsigned(f));
+    // slot / per and the rest: the product's upper half is the quotient or,
+    // where slot x per passes 2^32, at most one more.
+    int cc = int(slot), rr = 0;
+    if (per > 1) {
+        cc = int((static_cast<unsigned long long>(slot) * magic) >> 32);
+        rr = int(slot) - cc * per;
+        if (rr < 0) --cc, rr += per;
+    }
+    const int shift = 31 - __builtin_clz(unsigned(f));
     return {int(xcd >> shift) + (8 >> shift) * rr, int(xcd & unsigned(f - 1)) + f * cc};
 }
 

@@ -225,8 +225,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
     // Loader i's load j fills slots 64 (i + 4 j) + lane of a stage: A hi, A lo,
     // then W rows; 64 / SL rows each. A rows past M repeat row M - 1 and are
     // never stored.
-    const char* base[kLoads];   // wave-uniform
-    size_t offset[kLoads];      // 64 bits: the rows of a tile may lie more than 4 GiB apart
+    const char* base[kLoads];  // wave-uniform
+    size_t offset[kLoads];     // 64 bits: the rows of a tile may lie more than 4 GiB apart
     auto load_addresses = [&] {
         const int loader = wave - T::kMma;
 #pragma unroll
@@ -239,10 +239,10 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
                 const int r0 = r - lane / SL;
                 const int first = EPI == kSwiglu ? (r0 < BN / 2 ? n0 / 2 : N / 2 + n0 / 2 - BN / 2) : n0;
                 base[j] = reinterpret_cast<const char*>(W + size_t(first) * K + kz);
-                offset[j] = 2 * (size_t(r) * K + 8 * p);
+                offset[j] = 2 * (size_t(unsigned(r)) * unsigned(K) + unsigned(8 * p));
             } else {
                 base[j] = reinterpret_cast<const char*>((q0 >= kPlane ? Al : Ah) + size_t(m0) * K + kz);
-                offset[j] = 2 * (size_t(min(r, M - 1 - m0)) * K + 8 * p);
+                offset[j] = 2 * (size_t(unsigned(min(r, M - 1 - m0))) * unsigned(K) + unsigned(8 * p));
             }
         }
     };

@@ -27,9 +27,6 @@ extern "C" long long wrong_tiles(int M, int N, int BM, int BN) {
     for (const unsigned char s : seen) wrong += s != 1;
     return wrong;
 }
-extern "C" unsigned divide(unsigned slot, unsigned per) {
-    return map_divide(slot, per, unsigned(((1ull << 32) + per - 1) / per));
-}
 '''
 
 
@@ -41,7 +38,6 @@ def shim(tmp_path_factory):
                     str(where / 'shim.cpp'), '-o', str(where / 'shim.so')], check=True)
     lib = ctypes.CDLL(str(where / 'shim.so'))
     lib.wrong_tiles.restype = ctypes.c_longlong
-    lib.divide.restype = ctypes.c_uint
     return lib
 
 
@@ -57,10 +53,3 @@ def test_every_tile_once_of_the_largest(shim, m, n, bm, bn):
     """Rows up to the launch limit of the kernel that splits the operand (2^32
     threads of 256 per row), with outputs of 146 and 262 GB."""
     assert shim.wrong_tiles(m, n, bm, bn) == 0
-
-
-def test_divide(shim):
-    for per in (2, 3, 5, 7, 11, 1000, 16111, 16383, 16384, 65535, 131071):
-        for slot in [*range(0, 3 * per if per < 100 else 5), per - 1, per, per + 1, 2**31 - 1, 2**32 - 1,
-                     *(per * k + d for k in (17, 1001, 2**31 // per, (2**32 - 1) // per) for d in (-1, 0))]:
-            assert shim.divide(ctypes.c_uint(slot), ctypes.c_uint(per)) == slot // per, (slot, per)
