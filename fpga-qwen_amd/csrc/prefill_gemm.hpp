@@ -183,13 +183,19 @@ struct GemmArgs {
     unsigned magic;
 };
 
-// gate * sigmoid(gate) * up with sigmoid(g) = 0.5 + 0.5 tanh(g / 2)
-// (engine/core.cpp:636-639) from one exp2 and one correctly rounded division:
-// within 2 ulp of the exact sigmoid where it is not tiny, and exp2's argument
-// rounding (2^-24 |g|, relative) where it is, against the 2^-25 absolute of
-// the tanh form.
+// gate * sigmoid(gate) * up (engine/core.cpp:636-639) with e = exp(-|g|) <= 1 and
+// sigmoid(g) = 1 / (1 + e), or e / (1 + e) for g < 0. One quotient step on the
+// hardware reciprocal, with 1 + e carried as the two floats d + rest, rounds the
+// quotient once. Measured against 64 bits (rms relative, largest in ulp): gates of
+// standard deviation 0.64 3.03e-8, 2.6 ulp (0.5 + 0.5 tanh(g / 2), the reference's
+// form: 3.07e-8, 4.5; 1 / (1 + exp2), divided: 4.20e-8, 3.5); |g| < 0.5 2.88e-8, 1.06
+// (2.67e-8, 0.64; 4.28e-8, 2.1); -8 < g < -4, where the rounding of exp2's argument
+// (1.2 x 2^-24 |g|, relative) leads, 1.8e-7, 8.0 (9.1e-6, 513; 1.8e-7, 8.8).
 __device__ __forceinline__ float swiglu(float gate, float up) {
-    const float sig = 1.0f / (1.0f + __builtin_amdgcn_exp2f(gate * -1.4426950408889634f));
+    const float e = __builtin_amdgcn_exp2f(fabsf(gate) * -1.4426950408889634f);
+    const float d = 1.0f + e, rest = e - (d - 1.0f);
+    const float n = gate < 0.f ? e : 1.0f, inv = __builtin_amdgcn_rcpf(d), q = n * inv;
+    const float sig = __builtin_fmaf(inv, __builtin_fmaf(-rest, q, __builtin_fmaf(-d, q, n)), q);
     return gate * sig * up;
 }
 

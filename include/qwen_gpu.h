@@ -195,7 +195,7 @@ int qwen_gpu_op_gemm_static(const float* a, const uint16_t* w, float* c, int m, 
                             void* stream);
 /* Gate/up projection of the prefill path with its SwiGLU epilogue
  * (engine/core.cpp:630-639 with batch > 1: the gate and up projections, then
- * gate * (0.5 + 0.5 tanh(gate / 2)) * up): w natural FP16 [n x k] holding
+ * gate * sigmoid(gate) * up): w natural FP16 [n x k] holding
  * n / 2 gate rows then n / 2 up rows, a FP32 [m x k]; act[m][i] is written
  * as FP16 hi and lo planes [m x n / 2] and exponents act_exp [m x n / 16]
  * (one byte per group of 8 activations), with

@@ -97,17 +97,17 @@ def test_gemm_swiglu_against_fp64(qpkg, m, amp):
     ref = g * sig * u
     bg = 4e-6 * (np.abs(a64) @ np.abs(w64[:3072]).T) + 1e-7
     bu = 4e-6 * (np.abs(a64) @ np.abs(w64[3072:]).T) + 1e-7
-    # The last terms: the FP32 formula's own rounding, including 0.5 + 0.5 t
-    # for t near -1 (tanhf saturates to -1 below g ~ -17, where FP64 still
-    # has g sigmoid(g) u ~ 1e-8 g u): 2^-23 |g u| covers it.
+    # The last terms: the FP32 formula's own rounding (2^-23 |g u| also covers
+    # the reference's 0.5 + 0.5 tanh(g / 2) for tanh near -1).
     bound = (np.abs(sig * (1.0 + g * (1.0 - sig)) * u) * bg + np.abs(g * sig) * bu
              + 1e-6 * np.abs(ref) + 2.0 ** -23 * np.abs(g * u) + 1e-8)
     # The epilogue itself: the plain GEMM accumulates every element in the
     # same K order, so its g and u are the ones the SwiGLU epilogue saw. The
     # activation must be the reference formula evaluated in FP32 on them, up
-    # to the spread of two tanhf implementations and what FP16 hi + lo holds
-    # (2^-22 relative, half of FP16's subnormal spacing absolute). A hi / lo
-    # pair rounded from two different values misses this by an FP16 ulp.
+    # to what two evaluations of the sigmoid differ by (the reference's form
+    # rounds at 2^-24 absolute) and what FP16 hi + lo holds (2^-22 relative,
+    # half of FP16's subnormal spacing absolute). A hi / lo pair rounded from
+    # two different values misses this by an FP16 ulp.
     plain = qpkg.gemm(a, w)[rows]
     g32, u32 = plain[:, :3072], plain[:, 3072:]
     t32 = np.tanh(np.float32(0.5) * g32).astype(np.float32)
@@ -120,6 +120,44 @@ def test_gemm_swiglu_against_fp64(qpkg, m, amp):
     assert np.all(err <= bound), dict(ratio=float((err / bound).max()), row=int(rows[worst[0]]), col=int(worst[1]),
                                       g=float(g[worst]), u=float(u[worst]), got=float(got[worst]),
                                       ref=float(ref[worst]), bound=float(bound[worst]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('width', [0.5, 4.0, 16.0])
+def test_gemm_swiglu_sigmoid(qpkg, width):
+    """The sigmoid of the SwiGLU epilogue against FP64, without the GEMM's error:
+    one gate per row (A's column 0 times 1, exact), up a power of two. Half of
+    the results leave FP16 hi + lo unrounded (|lo| below a quarter of hi's
+    spacing); only those count. Relative to the result, in units of 2^-24: the
+    quotient and the product with the gate round once each (1), exp2 errs by
+    one ulp (2) and its argument by 1.22 |g| (its rounding, and that of
+    log2(e)), the last two times 1 - sigmoid. Around 0 the rms of three such
+    independent errors is 4.2e-8 (a rounding to nearest has 0.41 x 2^-24, over
+    one binade; exp2's ulp counts half); a further one, as of 1 + e, gives 4.9e-8."""
+    m, n, k = 8192, 256, 64
+    rng = np.random.default_rng(7)
+    step = 2.0 ** -19 * width  # 21 bits: hi + lo holds the gate exactly
+    gate = np.round(rng.uniform(-width, width, m) / step) * step
+    gate[np.abs(gate) < width / 64] = width / 64
+    sig = 1.0 / (1.0 + np.exp(-gate))
+    up = np.exp2(np.clip(6 - np.floor(np.log2(np.abs(gate * sig))), -14, 15))
+    a = np.zeros((m, k), np.float32)
+    a[:, 0], a[:, 1] = gate, up
+    assert np.array_equal(a[:, 0].astype(np.float64), gate)
+    w = np.zeros((n, k), np.float16)
+    w[:n // 2, 0] = 1
+    w[n // 2:, 1] = 1
+    act = qpkg.gemm_swiglu(a, w)
+    assert np.array_equal(act, np.repeat(act[:, :1], n // 2, 1))
+    act, ref = act[:, 0], gate * sig * up
+    lo = act - act.astype(np.float16).astype(np.float32)
+    kept = (np.abs(lo) < np.spacing(act.astype(np.float16)).astype(np.float32) / 4) & (np.abs(ref) > 1)
+    assert kept.mean() > 0.3
+    err = (np.abs(act - ref) / np.abs(ref) * 2.0 ** 24)[kept]
+    bound = (1 - sig) * (2 + 1.22 * np.abs(gate)) + 2.1
+    assert np.all(err <= bound[kept]), float((err / bound[kept]).max())
+    if width <= 0.5:
+        assert np.sqrt(np.mean(err ** 2)) * 2.0 ** -24 < 4.25e-8, float(np.sqrt(np.mean(err ** 2)) * 2.0 ** -24)
 
 
 def causal_attention_fp64(q, keys, values, pos0):
