@@ -45,7 +45,7 @@ template <int SPLITS>
 __device__ __forceinline__ float fold_splits(float x, const float* p, size_t stride) {
     static_assert(SPLITS == 0 || SPLITS == 4, "K-split GEMMs use 4 ranges");
     if constexpr (SPLITS == 0) return x;
-    else return x + (((p[0] + p[stride]) + p[2 * stride]) + p[3 * stride]);
+    else return x + ((p[0] + p[stride]) + (p[2 * stride] + p[3 * stride]));
 }
 
 
@@ -70,10 +70,10 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(float* __restrict__ X
         const size_t stride = size_t(rows) * kHidden / 4;
         const float4* pr = reinterpret_cast<const float4*>(parts + size_t(b) * kHidden) + tid;
         const float4 p0 = pr[0], p1 = pr[stride], p2 = pr[2 * stride], p3 = pr[3 * stride];
-        v4.x = v4.x + (((p0.x + p1.x) + p2.x) + p3.x);
-        v4.y = v4.y + (((p0.y + p1.y) + p2.y) + p3.y);
-        v4.z = v4.z + (((p0.z + p1.z) + p2.z) + p3.z);
-        v4.w = v4.w + (((p0.w + p1.w) + p2.w) + p3.w);
+        v4.x = v4.x + ((p0.x + p1.x) + (p2.x + p3.x));
+        v4.y = v4.y + ((p0.y + p1.y) + (p2.y + p3.y));
+        v4.z = v4.z + ((p0.z + p1.z) + (p2.z + p3.z));
+        v4.w = v4.w + ((p0.w + p1.w) + (p2.w + p3.w));
         *xr = v4;
     }
     const float v[4] = {v4.x, v4.y, v4.z, v4.w};
@@ -588,7 +588,9 @@ using Tile48x128 = GemmTile<48, 128, 4, 1, 5>;
 using Tile64x128 = GemmTile<64, 128, 4, 2, 5, 64, 8>;
 using Tile96x128 = GemmTile<96, 128, 4, 2, 4, 64, 8>;
 using Tile128x128 = GemmTile<128, 128, 2, 4, 3, 64, 8>;
-using Fold128x128 = GemmTile<128, 128, 2, 4, 3>;  // the sums of the ranges take the registers of 8 loaders
+// Folding: the sums of the ranges take the registers of 8 loaders.
+using Fold96x128 = GemmTile<96, 128, 4, 2, 4>;
+using Fold128x128 = GemmTile<128, 128, 2, 4, 3>;
 using Tile64x192 = GemmTile<64, 192, 2, 4, 4>;
 using Tile96x192 = GemmTile<96, 192, 3, 2, 3>;
 using Tile128x192 = GemmTile<128, 192, 2, 4, 2>;
@@ -705,7 +707,7 @@ void project_residual(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W,
     else if (GemmMap(rows, kHidden, 64, 128, 1).rounds() == 1)
         launch<Tile64x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
     else if (GemmMap(rows, kHidden, 96, 128, 1).rounds() == 1)
-        launch<Tile96x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
+        launch<Fold96x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
     else
         launch<Fold128x128, kWhole>(Ah, Al, W, x, rows, kHidden, K, stream, 1, ep);
 }

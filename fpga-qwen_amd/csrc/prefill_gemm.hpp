@@ -101,7 +101,7 @@ __device__ __forceinline__ double lane_xor32(double v) {
 
 // kParts: the partial products of K range blockIdx.z, stored at C + blockIdx.z
 // M N. kFold: the 4 K ranges one after the other in one workgroup, each summed
-// from zero, ((p0 + p1) + p2) + p3 added into C: the sum that the row kernels
+// from zero, (p0 + p1) + (p2 + p3) added into C: the sum that the row kernels
 // form from kParts' ranges. Guarded: with the range guard of the down GEMM.
 enum GemmKind { kStore, kParts, kPartsGuarded, kFold, kFoldGuarded, kSwiglu, kQkv };
 constexpr int kKRanges = 4;
@@ -252,12 +252,13 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
             }
         }
     };
-    auto issue = [&](int kt) {
-        unsigned char* stage = smem + (kt % NS) * kStageBytes + 1024 * (wave - T::kMma);
+    auto issue_to = [&](int kt, int buffer) {
+        unsigned char* stage = smem + buffer * kStageBytes + 1024 * (wave - T::kMma);
 #pragma unroll
         for (int j = 0; j < kLoads; ++j)
             load_lds16(base[j] + offset[j] + size_t(kt) * (2 * TK), stage + 1024 * T::kLoaders * j);
     };
+    auto issue = [&](int kt) { issue_to(kt, kt % NS); };
     // Waits until at most `later` whole stages of this loader's are pending.
     auto wait_stages = [&](int later) {
         if (later >= NS - 1) {
@@ -283,9 +284,10 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
             else flagged |= flags[blockIdx.z];
         }
     }
-    // Stages of a K range of kFold, and the sum of the ranges so far.
+    // Stages of a K range of kFold; range 0 or 2, and the sum of ranges 0 and 1, in
+    // the end of all.
     const int range = nk / kKRanges;
-    floatx4 total[kIsFold ? TN : 1][kIsFold ? TM : 1];
+    floatx4 even[kIsFold ? TN : 1][kIsFold ? TM : 1], total[kIsFold ? TN : 1][kIsFold ? TM : 1];
 
     floatx4 acc[TN][TM];
     auto clear = [&] {
@@ -326,22 +328,15 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
         }
     };
 
-    // kFold: range z of `range` stages is complete; its sum, scaled by `scale(t)`,
-    // joins the total.
-    auto fold_range = [&](int z, auto&& scale) {
+    // kFold: a range is complete; its sums, scaled by `scale(t)`, join the others.
+    auto each_sum = [&](auto&& scale, auto&& join) {
         if constexpr (kIsFold) {
 #pragma unroll
             for (int t = 0; t < TM; ++t) {
                 const float sc = scale(t);
 #pragma unroll
-                for (int i = 0; i < TN; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float p = acc[i][t][e] * sc;
-                        total[i][t][e] = z == 0 ? p : total[i][t][e] + p;
-                    }
+                for (int i = 0; i < TN; ++i) join(i, t, acc[i][t] * sc);
             }
-            clear();
         }
     };
     auto one = [](int) { return 1.f; };
@@ -386,7 +381,10 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
         for (int kt = 0; kt < nk; ++kt) {
             if constexpr (kIsFold) {
                 if (kt == range_end) {
-                    fold_range(z++, one);
+                    if (z % 2 == 0) each_sum(one, [&](int i, int t, floatx4 p) { even[i][t] = p; });
+                    else each_sum(one, [&](int i, int t, floatx4 p) { total[i][t] = even[i][t] + p; });
+                    clear();
+                    ++z;
                     range_end += range;
                 }
             }
@@ -419,7 +417,7 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
             }
         }
         wait_lgkm0();
-        fold_range(z, one);
+        each_sum(one, [&](int i, int t, floatx4 p) { total[i][t] = total[i][t] + (even[i][t] + p); });
     }
 
     // Guarded down GEMM: the loop again with each A group rescaled in LDS to its
@@ -435,13 +433,25 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
             auto range_scale = [&](int z) {
                 return [&, z](int t) { return pow2(row_flag(m0 + (wm * TM + t) * 16 + row, z)); };
             };
+            // kFold: the sum of ranges 0 and 1 waits in LDS behind the one stage
+            // (the loaders' addresses, live in this loop, leave no registers).
+            static_assert(!kIsFold || kStageBytes + 4 * BM * BN <= kSmem, "parked sums");
+            auto parked = [&](int i, int t) -> floatx4& {
+                return *reinterpret_cast<floatx4*>(smem + kStageBytes + 16 * ((TN * t + i) * 64 * T::kMma + tid));
+            };
             for (int kt = 0; kt < nk; ++kt) {
                 const int z = kIsFold ? kt / range : int(blockIdx.z);
-                if (kIsFold && mma && kt > 0 && kt % range == 0) fold_range(z - 1, range_scale(z - 1));
+                if (kIsFold && mma && kt > 0 && kt % range == 0) {
+                    each_sum(range_scale(z - 1), [&](int i, int t, floatx4 p) {
+                        if (z == 2) parked(i, t) = even[i][t] + p;
+                        else even[i][t] = p;
+                    });
+                    clear();
+                }
                 stage_barrier();  // every wave is done with the stage before (all loads were waited for)
-                unsigned char* stage = smem + (kt % NS) * kStageBytes;
+                unsigned char* stage = smem;
                 if (!mma) {
-                    issue(kt);
+                    issue_to(kt, 0);
                     wait_vmcnt<0>();
                 }
                 stage_barrier();
@@ -483,7 +493,9 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
                     wait_lgkm0();
                 }
             }
-            if (mma) fold_range(kKRanges - 1, range_scale(kKRanges - 1));
+            if (kIsFold && mma)
+                each_sum(range_scale(kKRanges - 1),
+                         [&](int i, int t, floatx4 p) { total[i][t] = parked(i, t) + (even[i][t] + p); });
         }
     }
     stage_barrier();  // every wave is done with the ring: the results are staged over it

@@ -10,6 +10,7 @@ the oracle gate and the reuse-equals-fresh invariant
 (tools/check_native_cpu_prefix.py).
 """
 import json
+import shutil
 from pathlib import Path
 
 import numpy as np
@@ -407,6 +408,44 @@ def test_attention_prefill_head_split(qpkg, rows, end):
     whole = qpkg.attention_prefill(qkv, keys, values, 0)
     got = qpkg.attention_prefill(qkv[end - rows:end], keys[:, :end], values[:, :end], end - rows)
     assert np.array_equal(got.view(np.uint32), whole[end - rows:end].view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_prefill_fold_order(qpkg, pack0, tmp_path):
+    """O and down add their 4 K ranges as (p0 + p1) + (p2 + p3), in the row
+    kernels (up to 1024 rows) and in the folding GEMMs (64-, 96- and 128-row
+    tiles). Layer 0 is built for exact partials: all queries and keys 0, so
+    every score is 0, all values 1, so the attention output is 1, and O rows of
+    even channels 1024, 2^-14, 2^-14 and -1024 in the four ranges. In pairs that
+    is 2^-14; 1024 + 2^-14 is a tie that rounds to 1024, so one after the other
+    it is 0. Nothing else adds to the residual, which starts at 1."""
+    path = tmp_path / 'weights.bin'
+    shutil.copyfile(pack0, path)
+    shutil.copyfile(str(pack0) + '.index', str(path) + '.index')
+    blob = np.memmap(path, np.uint8, 'r+')
+    tensors = {}
+    for line in Path(str(path) + '.index').read_text().splitlines()[1:]:
+        name, kind, rows, cols, offset, length = line.split()
+        if kind == 'F16':
+            tensors[name] = blob[int(offset):int(offset) + int(length)].view('<f2').reshape(int(rows), int(cols))
+    for layer in range(28):
+        tensors[f'model.layers.{layer}.self_attn.o_proj.weight'][:] = 0
+        tensors[f'model.layers.{layer}.mlp.down_proj.weight'][:] = 0
+    first = 'model.layers.0.self_attn.'
+    for name in ('q', 'k', 'v'):
+        tensors[first + name + '_proj.weight'][:] = 0
+    tensors[first + 'v_proj.weight'][:, 0] = 1
+    tensors[first + 'o_proj.weight'][::2, ::512] = [1024, 2.0 ** -14, 2.0 ** -14, -1024]
+    tensors['model.embed_tokens.weight'][0] = 1
+    blob.flush()
+    del tensors, blob
+    with qpkg.Model(path) as m:
+        for rows in (2, 85, 1024, 1100, 2100, 3100):
+            m.reset()
+            m.prefill([0] * rows)
+            hidden = m.hidden().astype(np.float64)
+            assert np.allclose(hidden[::2] / hidden[1], 1 + 2.0 ** -14, rtol=2.0 ** -22, atol=0), rows
+            assert np.all(hidden[1::2] == hidden[1]), rows
 
 
 @pytest.mark.gpu
