@@ -315,8 +315,8 @@ def test_prefill_rows_independent_of_grouping(qpkg, pack0):
 @pytest.mark.gpu
 @pytest.mark.parametrize('n,k', [(1024, 1024), (4096, 1024), (1024, 3072), (6144, 64)])
 def test_gemm_tile_edges(qpkg, n, k):
-    """Row counts at the edges of every tile height (16, 32, 64, 128) and of
-    the rounds that choose between them: each call's rows must be the bits of
+    """Row counts at the edges of every tile height (16, 32, 48, 64, 96, 128) and
+    of the rounds that choose between them: each call's rows must be the bits of
     one 700-row call (whatever tile either takes, every element adds its K
     terms in one order), which in turn meets the FP64 bound. K = 64 is a
     single LDS stage."""
@@ -326,7 +326,8 @@ def test_gemm_tile_edges(qpkg, n, k):
     full = qpkg.gemm(a, w)
     bound = 4e-6 * (np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T) + 1e-7
     assert np.all(np.abs(full - a.astype(np.float64) @ w.astype(np.float64).T) <= bound)
-    for m in (1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 513):
+    for m in (1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 96, 97, 127, 128, 129, 143, 144, 145, 191, 192, 193,
+              255, 256, 257, 288, 289, 321, 481, 513, 576, 577):
         first = (37 * m) % (700 - m)
         got = qpkg.gemm(a[first:first + m], w)
         assert np.array_equal(got.view(np.uint32), full[first:first + m].view(np.uint32)), m
@@ -335,24 +336,28 @@ def test_gemm_tile_edges(qpkg, n, k):
 @pytest.mark.gpu
 def test_gemm_swiglu_tile_edges(qpkg):
     """The same for the SwiGLU epilogue (gate and up columns of one tile), with
-    rows whose activations carry exponents among them."""
+    rows whose activations carry exponents among them. Tiles of 16 x 32 (up to
+    16 rows) to 128 x 192 (641), 128 x 256 (1025) and 96 x 192 (1281 to 1536)."""
     rng = np.random.default_rng(61)
-    a = rng.standard_normal((1300, 1024), dtype=np.float32)
+    a = rng.standard_normal((1500, 1024), dtype=np.float32)
     a[::5] *= np.float32(300)
     w = (rng.standard_normal((6144, 1024), dtype=np.float32) * 0.02).astype(np.float16)
     full, exps = qpkg.gemm_swiglu(a, w, exponents=True)
     assert exps.any() and not exps.all() and np.isfinite(full).all()
-    for m in (1, 16, 17, 32, 33, 64, 65, 128, 129, 320, 321, 640, 641, 1024, 1025):
-        first = (37 * m) % (1300 - m)
+    for m in (1, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 144, 145, 192, 193, 256, 257, 288, 289, 320, 321, 480, 481, 640,
+              641, 1024, 1025, 1281, 1344, 1345):
+        first = (37 * m) % (1500 - m)
         got, e = qpkg.gemm_swiglu(a[first:first + m], w, exponents=True)
         assert np.array_equal(got.view(np.uint32), full[first:first + m].view(np.uint32)), m
         assert np.array_equal(e, exps[first:first + m]), m
 
 
 @pytest.mark.gpu
-def test_prefill_rows_independent_of_tile(qpkg, pack0):
-    """The QKV epilogue (a head per tile of 16, 32, 64 or 128 rows) and the
-    K-split GEMMs: calls of 2 to 300 rows leave the logits of one 700-row
+@pytest.mark.parametrize('calls', [(2, 16, 17, 33, 65, 130, 137, 300), (96, 200, 404), (144, 556)])
+def test_prefill_rows_independent_of_tile(qpkg, pack0, calls):
+    """The QKV epilogue (a head per tile of 16 rows up to 128, of 32 up to 256, 48
+    up to 384, 64 up to 512, 96 up to 576, then 128) and the K-split GEMMs (tiles of
+    16 x 32 to 128 x 128, each in one of these calls): the logits of one 700-row
     call."""
     prompt = PROMPTS['long_3968'][:700]
     with qpkg.Model(pack0) as m:
@@ -360,7 +365,7 @@ def test_prefill_rows_independent_of_tile(qpkg, pack0):
         whole = m.logits().view(np.uint32).copy()
         m.reset()
         at = 0
-        for rows in (2, 16, 17, 33, 65, 130, 137, 300):
+        for rows in calls:
             m.prefill(prompt[at:at + rows])
             at += rows
         assert at == 700
@@ -449,11 +454,11 @@ def test_prefill_fold_order(qpkg, pack0, tmp_path):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('rows', [1100, 2100])
+@pytest.mark.parametrize('rows', [1100, 2100, 3100])
 def test_prefill_folding_gemms(qpkg, pack0, rows):
     """Beyond 1024 rows the O and down GEMMs add their 4 K ranges themselves
-    (64-row tiles, then 128-row tiles from 2049 rows): the bits of calls of at
-    most 1024 rows, whose ranges the row kernels add."""
+    (64-row tiles, 96-row tiles from 2049 rows, 128-row tiles from 3073): the
+    bits of calls of at most 1024 rows, whose ranges the row kernels add."""
     prompt = PROMPTS['long_3968'][:rows]
     with qpkg.Model(pack0) as m:
         m.prefill(prompt)
@@ -467,22 +472,25 @@ def test_prefill_folding_gemms(qpkg, pack0, rows):
 @pytest.mark.gpu
 def test_prefill_folding_gemms_range_guard(qpkg, tmp_path):
     """The same with activations past FP16's range (norm gains of 32768 in 8
-    channels): the folding down GEMM rescales each K range of a flagged row by
-    that range's exponent, as the ranged one does."""
+    channels): the folding down GEMM, with tiles of 64, 96 and 128 rows, rescales
+    each K range of a flagged row by that range's exponent, as the ranged one
+    does."""
     import test_export
     path = test_export.write_full_checkpoint(tmp_path / 'model.safetensors', gains=test_export.LARGE_GAINS)
     out = tmp_path / 'pack' / 'weights.bin'
     test_export.export_pack.write_pack(path, out)
     path.unlink()
-    prompt = PROMPTS['long_3968'][:1100]
-    with qpkg.Model(out, context=1200) as m:
-        m.prefill(prompt)
-        whole = m.logits().view(np.uint32).copy()
-        assert np.isfinite(whole.view(np.float32)).all()
-        m.reset()
-        m.prefill(prompt[:500])
-        m.prefill(prompt[500:])
-        assert np.array_equal(m.logits().view(np.uint32), whole)
+    with qpkg.Model(out, context=3200) as m:
+        for rows in (1100, 2100, 3100):
+            prompt = PROMPTS['long_3968'][:rows]
+            m.reset()
+            m.prefill(prompt)
+            whole = m.logits().view(np.uint32).copy()
+            assert np.isfinite(whole.view(np.float32)).all()
+            m.reset()
+            for at in range(0, rows, 500):
+                m.prefill(prompt[at:at + 500])
+            assert np.array_equal(m.logits().view(np.uint32), whole), rows
 
 
 @pytest.mark.gpu
