@@ -531,14 +531,11 @@ void Engine::run_append(const int* ids, size_t count) {
         std::copy(ids, ids + batched, ids_host_);
         HIP_CHECK(hipMemcpyAsync(ids_dev_, ids_host_, batched * sizeof(int), hipMemcpyHostToDevice, stream_));
         const int rows = int(batched);
-        float* final_row = launch_prefill_chunk(prefill_layers_.data(), embed_, ids_dev_, rows, pos_, cosines_, sines_,
-                                                options_.context, prefill_, stream_);
+        launch_prefill_chunk(prefill_layers_.data(), embed_, ids_dev_, rows, pos_, cosines_, sines_, options_.context,
+                             prefill_, scratch_.x, stream_);
         pos_ += rows;
-        if (batched == count) {
-            DecodeScratch head = scratch_;
-            head.x = final_row;
-            launch_lm_head(lm_t_, final_norm_, head, result_host_, next_tag(), stream_, ++result_seq_);
-        }
+        if (batched == count)
+            launch_lm_head(lm_t_, final_norm_, scratch_, result_host_, next_tag(), stream_, ++result_seq_);
     }
     if (batched < count) run_token(ids[count - 1], true, 0);
     HIP_CHECK(hipGetLastError());

@@ -40,15 +40,6 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const int* __restrict__
     for (int j = threadIdx.x; j < kHidden; j += 256) X[size_t(b) * kHidden + j] = h2f(row[j]);
 }
 
-// x + the SPLITS partial products of a K-split GEMM in a fixed order.
-template <int SPLITS>
-__device__ __forceinline__ float fold_splits(float x, const float* p, size_t stride) {
-    static_assert(SPLITS == 0 || SPLITS == 4, "K-split GEMMs use 4 ranges");
-    if constexpr (SPLITS == 0) return x;
-    else return x + ((p[0] + p[stride]) + (p[2 * stride] + p[3 * stride]));
-}
-
-
 // out[b] = RMSNorm(x[b]) (engine/core.cpp:207-215): FP32 squares, FP64 sum,
 // written as the FP16 hi / lo planes of the next GEMM's A operand, split as
 // out * 2^-row_exp[b] (split_exponent of the row's largest magnitude; 0
@@ -565,12 +556,12 @@ __global__ __launch_bounds__(256 * HEADS) void attn_prefill_mfma_kernel(const fl
     }
 }
 
-// X[b] += the SPLITS partial products of a K-split GEMM (rows x 1024).
-template <int SPLITS>
-__global__ __launch_bounds__(256) void fold_rows_kernel(float* __restrict__ X, const float* __restrict__ parts,
-                                                        int rows) {
-    const size_t idx = size_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx < size_t(rows) * kHidden) X[idx] = fold_splits<SPLITS>(X[idx], parts + idx, size_t(rows) * kHidden);
+// out = x + the 4 partial products of a K-split GEMM, one row of 1024.
+__global__ __launch_bounds__(256) void fold_row_kernel(const float* __restrict__ x, const float* __restrict__ parts,
+                                                       float* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const float* p = parts + i;
+    out[i] = x[i] + ((p[0] + p[kHidden]) + (p[2 * kHidden] + p[3 * kHidden]));
 }
 
 // Tiles (by rows and outputs): MFMA wave grid (outputs x rows), LDS stages,
@@ -876,9 +867,9 @@ void launch_attention_prefill(const float* qkv, const uint16_t* keys, const uint
                                                                  scale);
 }
 
-float* launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, const int* ids_dev, int rows, int pos0,
-                            const float* cosines, const float* sines, int context, const PrefillScratch& s,
-                            hipStream_t stream) {
+void launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, const int* ids_dev, int rows, int pos0,
+                          const float* cosines, const float* sines, int context, const PrefillScratch& s,
+                          float* final_row, hipStream_t stream) {
     require(rows >= 1 && rows <= kPrefillRows, "prefill chunk: bad row count");
     embed_rows_kernel<<<rows, 256, 0, stream>>>(ids_dev, embed, s.x);
     // Where the O and down GEMMs leave their 4 K ranges apart, the row kernel
@@ -933,8 +924,7 @@ float* launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, c
         if (l + 1 < kLayers) finish_layer(L, s, rows, pos0);
         else finish_layer(L, last, 1, pos0 + rows - 1);
     }
-    fold_rows_kernel<kKRanges><<<kHidden / 256, 256, 0, stream>>>(last.x, last.part, 1);
-    return last.x;
+    fold_row_kernel<<<kHidden / 256, 256, 0, stream>>>(last.x, last.part, final_row);
 }
 
 }  // namespace qwen_hip

@@ -70,10 +70,10 @@ void launch_attention_prefill(const float* qkv, const uint16_t* keys, const uint
                               uint16_t* att_lo, int rows, int pos0, int context, hipStream_t stream);
 
 // All 28 layers for `rows` prompt ids (device) at positions pos0..pos0+rows-1:
-// K/V land in the cache. Returns the final residual row of the last position
-// (in s.x; the other rows of s.x stop short of the last layer).
-float* launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, const int* ids_dev, int rows, int pos0,
-                            const float* cosines, const float* sines, int context, const PrefillScratch& s,
-                            hipStream_t stream);
+// K/V land in the cache, the final residual row of the last position in
+// final_row [1024] (the rows of s.x stop short of the last layer).
+void launch_prefill_chunk(const PrefillLayer* layers, const uint16_t* embed, const int* ids_dev, int rows, int pos0,
+                          const float* cosines, const float* sines, int context, const PrefillScratch& s,
+                          float* final_row, hipStream_t stream);
 
 }  // namespace qwen_hip
