@@ -46,11 +46,15 @@ __device__ __forceinline__ void load_lds16(const void* src, unsigned char* lds) 
 // the parts apart and waits for every load it knows of before an LDS read.
 // base and lds (an LDS byte address) wave-uniform, offset in bytes per lane.
 // The caller waits (wait_vmcnt) before the data is read; the compiler's own
-// counted waits only become stricter by the loads it does not see.
+// counted waits only become stricter by the loads it does not see. M0 is a
+// register that the compiler reserves, so its value is put back.
 __device__ __forceinline__ void load_lds16_opaque(const void* base, unsigned offset, unsigned lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
-                 : "memory", "m0");
+    unsigned m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0)
+                 : "s"(lds), "v"(offset), "s"(base)
+                 : "memory");
 #endif
 }
 __device__ __forceinline__ unsigned lds_address(const unsigned char* p) {
