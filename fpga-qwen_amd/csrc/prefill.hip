@@ -482,6 +482,7 @@ __global__ __launch_bounds__(256 * HEADS) void attn_prefill_mfma_kernel(const fl
     } else {
         for (int step = 0; step + 1 < nsteps; ++step) {
             wait_vmcnt<0>();  // this wave's loads of K tile step + 1 and V tile step
+            wait_lgkm0();     // and its reads of K tile step (MFMAs that need them may be moved)
             phase_barrier();
             // K buffer step and V buffer step - 1 have been read by both waves.
             issue(keys, step + 2, 0);
@@ -497,6 +498,7 @@ __global__ __launch_bounds__(256 * HEADS) void attn_prefill_mfma_kernel(const fl
         }
     }
     wait_vmcnt<0>();
+    wait_lgkm0();
     phase_barrier();
     if (has(nsteps - 1)) vector_phase(nsteps - 1);
     wait_lgkm0();
