@@ -324,7 +324,7 @@ void Engine::init_state() {
     ps.att_lo = device_alloc<uint16_t>(prows * kQDim);
     ps.act_hi = device_alloc<uint16_t>(prows * kFFN);
     ps.act_lo = device_alloc<uint16_t>(prows * kFFN);
-    ps.part = device_alloc<float>(4 * prows * kHidden);
+    ps.part = device_alloc<float>(4 * std::min(prows, size_t(kFoldRows)) * kHidden);
     ps.row_exp = device_alloc<int>(prows);
     ps.act_flag = device_alloc<int>(4 * prows);
     ps.act_exp = device_alloc<uint8_t>(prows * (kFFN / 8));

@@ -689,7 +689,7 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
 // 3072 rows 47.3 / 60.6 and 33.1 / 46.8 (128 x 128 tiles; 96 x 128 take 27.6 where
 // those take 33.6); at 1024 rows 19.4 / 23.6 and 21.5 / 27.9. Whole
 // prefills of 3500 rows 12.18 -> 11.20 ms, of 3968 rows 13.47 -> 12.51.
-bool gemm_folds(int rows) { return rows > 1024; }
+bool gemm_folds(int rows) { return rows > kFoldRows; }
 
 template <bool kGuarded>
 void project_residual(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* x, float* parts, int rows, int K,

@@ -22,6 +22,10 @@ struct PrefillLayer {
     uint16_t* values;          // [8][context][128]
 };
 
+// Calls of more rows add the K ranges of their O and down GEMMs in the GEMM and
+// need no partial products.
+inline constexpr int kFoldRows = 1024;
+
 // Activations of one batched pass (up to kPrefillRows rows each). GEMM
 // inputs are kept as FP16 hi / lo planes (hi = fp16(v), lo = fp16(v - hi)).
 struct PrefillScratch {
@@ -33,7 +37,7 @@ struct PrefillScratch {
     uint16_t* att_lo;
     uint16_t* act_hi;   // [rows x 3072] SwiGLU output
     uint16_t* act_lo;
-    float* part;        // [4 x rows x 1024] K-split partial products of the O and down GEMMs
+    float* part;        // [4 x min(rows, kFoldRows) x 1024] partial products of the O and down GEMMs' K ranges
     // Range guard of the FP16 split (values from 65504 up do not fit FP16):
     int* row_exp;       // [rows] the normalized row was split as h * 2^-row_exp
     int* act_flag;      // [rows x 4] largest SwiGLU group exponent per K range of the down GEMM

@@ -9,6 +9,7 @@ chunk size (needed for exact canonical prefix reuse), and end to end through
 the oracle gate and the reuse-equals-fresh invariant
 (tools/check_native_cpu_prefix.py).
 """
+import ctypes
 import json
 import shutil
 from pathlib import Path
@@ -513,3 +514,26 @@ def test_gemm_rows_far_apart(qpkg):
     qpkg._check(lib.qwen_gpu_op_gemm(ad.ptr, wd.ptr, cd.ptr, 1, n, k, 0, None))
     qpkg.synchronize()
     assert np.array_equal(cd.to_array(np.float32, n), np.arange(1, n + 1, dtype=np.float32))
+
+
+@pytest.mark.gpu
+def test_sequence_memory(qpkg, pack0):
+    """Device memory of one further sequence at 4096 positions: 448 MiB of K/V and
+    44 KiB per prefill row (176 MiB), partial products for 1024 rows only (16
+    MiB), and a few MiB of logits and exchange words."""
+    def free():
+        left, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert qpkg.load_library().hipMemGetInfo(ctypes.byref(left), ctypes.byref(total)) == 0
+        return left.value
+    # The runtime may hand out memory that it kept from earlier frees: the
+    # largest of three.
+    with qpkg.Model(pack0, context=16) as owner:
+        sequences, used = [], []
+        for _ in range(3):
+            before = free()
+            sequences.append(owner.share(context=4096))
+            used.append((before - free()) / 2 ** 20)
+        for sequence in sequences:
+            sequence.close()
+    print(used)
+    assert max(used) < 665, used
