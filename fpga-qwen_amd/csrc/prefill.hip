@@ -576,7 +576,6 @@ using Tile48x64 = GemmTile<48, 64, 2, 3, 7>;
 using Tile64x64 = GemmTile<64, 64, 2, 4, 6, 64, 8>;
 using Tile48x96 = GemmTile<48, 96, 3, 1, 6>;
 using Tile64x96 = GemmTile<64, 96, 3, 2, 5>;
-using Tile96x96 = GemmTile<96, 96, 3, 2, 4>;
 using Tile48x128 = GemmTile<48, 128, 4, 1, 5>;
 using Tile64x128 = GemmTile<64, 128, 4, 2, 5, 64, 8>;
 using Tile96x128 = GemmTile<96, 128, 4, 2, 4, 64, 8>;
@@ -584,7 +583,6 @@ using Tile128x128 = GemmTile<128, 128, 2, 4, 3, 64, 8>;
 // Folding: the sums of the ranges take the registers of 8 loaders.
 using Fold96x128 = GemmTile<96, 128, 4, 2, 4>;
 using Fold128x128 = GemmTile<128, 128, 2, 4, 3>;
-using Tile64x192 = GemmTile<64, 192, 2, 4, 4>;
 using Tile96x192 = GemmTile<96, 192, 3, 2, 3>;
 using Tile128x192 = GemmTile<128, 192, 2, 4, 2>;
 using Tile128x256 = GemmTile<128, 256, 4, 2, 2>;
@@ -666,8 +664,6 @@ void gemm(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C, i
         if constexpr (EPI == kSwiglu) {
             consider.template operator()<Tile48x96>(11.9);
             consider.template operator()<Tile64x96>(13.2);
-            consider.template operator()<Tile96x96>(16.3);
-            consider.template operator()<Tile64x192>(18.5);
             consider.template operator()<Tile96x192>(25.8);
             consider.template operator()<Tile128x192>(29.2);
         }
