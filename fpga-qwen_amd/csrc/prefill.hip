@@ -708,15 +708,16 @@ void project_residual(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W,
 // -> 3.6 us), longer ones are read twice.
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, uint16_t* __restrict__ hi,
                                                          uint16_t* __restrict__ lo, int* __restrict__ row_exp, int K) {
+    typedef float piece __attribute__((ext_vector_type(4), aligned(4)));  // A is the caller's: floats, not vectors
     constexpr int kHeld = 4;  // 4-column pieces per thread
     const size_t base = size_t(blockIdx.x) * K;
     const int tid = threadIdx.x, pieces = K / 4;
-    const floatx4* row = reinterpret_cast<const floatx4*>(A + base);
+    const piece* row = reinterpret_cast<const piece*>(A + base);
     floatx4 held[kHeld];
     float big = 0.f;
     auto grow = [&](floatx4 v) { big = fmaxf(fmaxf(big, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3]))); };
 #pragma unroll
-    for (int k = 0; k < kHeld; ++k) held[k] = tid + 256 * k < pieces ? row[tid + 256 * k] : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < kHeld; ++k) held[k] = tid + 256 * k < pieces ? floatx4(row[tid + 256 * k]) : floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < kHeld; ++k) grow(held[k]);
     for (int i = tid + 256 * kHeld; i < pieces; i += 256) grow(row[i]);

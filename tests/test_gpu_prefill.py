@@ -517,6 +517,25 @@ def test_gemm_rows_far_apart(qpkg):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('m,k', [(3, 64), (37, 1024), (5, 4160)])
+def test_gemm_operand_alignment(qpkg, m, k):
+    """A may begin at any float: the bits of the call whose A begins on 16 bytes,
+    through the entry that allocates and the one that does not (rows held in
+    registers up to 4096 columns, read twice beyond)."""
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    w = (rng.standard_normal((128, k), dtype=np.float32) * 0.02).astype(np.float16)
+    expected = qpkg.gemm(a, w).view(np.uint32)
+    wd, cd, lib = qpkg.DeviceBuffer.from_array(w), qpkg.DeviceBuffer(m * 128 * 4), qpkg.load_library()
+    for shift in (1, 2, 3):
+        ad = qpkg.DeviceBuffer.from_array(np.r_[np.full(shift, np.nan, np.float32), a.ravel()])
+        for entry in (lib.qwen_gpu_op_gemm, lib.qwen_gpu_op_gemm_static):
+            qpkg._check(entry(ad.ptr.value + 4 * shift, wd.ptr, cd.ptr, m, 128, k, 0, None))
+            qpkg.synchronize()
+            assert np.array_equal(cd.to_array(np.uint32, m * 128).reshape(m, 128), expected), shift
+
+
+@pytest.mark.gpu
 def test_sequence_memory(qpkg, pack0):
     """Device memory of one further sequence at 4096 positions: 448 MiB of K/V and
     44 KiB per prefill row (176 MiB), partial products for 1024 rows only (16
