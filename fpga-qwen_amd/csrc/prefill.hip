@@ -602,17 +602,17 @@ void launch(const uint16_t* Ah, const uint16_t* Al, const uint16_t* W, float* C,
     gemm_kernel<T, EPI><<<dim3(map.groups(), 1, splits), T::kThreads, 0, stream>>>(args, ep);
 }
 
-// Every CU runs one workgroup at a time, so a launch takes as many rounds as
-// its fullest XCD has 32 workgroups; the tile with the least rounds x price is
-// taken. A price is the time of a full round of that tile, in us: of gate/up
-// (K 1024), of down (4 K ranges of 768; O, of 512, has the same order) and of QKV
-// (K 1024); a last round that leaves CUs idle is somewhat cheaper, more so for
-// the large tiles (QKV 128: 32 workgroups 14.5 us, 192 17.8 to 20, 256 21.9; gate/up
+// A launch takes as many rounds as its fullest XCD has 32 workgroups, one per CU
+// (of 16 x 32, two fit a CU: it is priced as if they did not); the tile with the
+// least rounds x price is taken. A price is the time of a full round of that tile, in
+// us: of gate/up (K 1024), of down (4 K ranges of 768; O, of 512, has the same order)
+// and of QKV (K 1024); a last round that leaves CUs idle is somewhat cheaper, more so
+// for the large tiles (QKV 128: 32 workgroups 14.5 us, 192 17.8 to 20, 256 21.9; gate/up
 // 64 x 64: 96 9.5, 192 10.8), as fewer CUs draw on the L2s, the memory and the
 // clock. Tiles of short prompts keep all CUs busy: one row tile of 128 x 128
 // would leave 208 of them idle in gate/up and run 19 us. Heights of 48 and 96
 // rows lie between the powers of two (whole prefill of 380 rows 2.10 -> 2.01 ms, of
-// 1300 rows 4.82 -> 4.44); not for the K ranges of O and down (700 rows: 96 x 128
+// 1300 rows 4.82 -> 4.44); 96 not for the K ranges of O and down (700 rows: 96 x 128
 // 13.5 / 17.3 us on all CUs, 128 x 128 on 192 of them 12.1 / 16.1, and the row kernel
 // behind them 7.5 instead of 5.7).
 template <int EPI>

@@ -143,8 +143,8 @@ struct GemmEpilogue {
 
 // Tile of a workgroup: BM activation rows x BN outputs, K in stages of TK
 // through a ring of NS LDS buffers. WN x WM waves run the MFMAs: wave (wn, wm)
-// holds the 16-output tiles wn TN .. and the 16-row tiles wm TM ... 4 more
-// waves, one per SIMD, only issue the direct global -> LDS loads: a CU accepts
+// holds the 16-output tiles wn TN .. and the 16-row tiles wm TM ... 4 or 8 more
+// waves, evenly on the SIMDs, only issue the direct global -> LDS loads: a CU accepts
 // 64 bytes of loads per clock, so a stage's loads hold up the waves that issue
 // them for about as long as the stage's MFMAs take, and waves that do both can
 // do neither during the other.
@@ -216,7 +216,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_kernel(const GemmArgs args, 
     static_assert(EPI != kSwiglu || TN % 2 == 0, "a wave of the SwiGLU epilogue holds gate and up tiles");
     // Results staged for the stores, over the ring: QKV rows (and the waves'
     // shares of the row sums), the SwiGLU planes or the C tile of the
-    // workgroup; pitches 16 bytes past a multiple of the banks.
+    // workgroup; pitches of an odd number of 16-byte slots, so that 16 rows begin in
+    // the 16 slots of a bank cycle.
     constexpr int kPitch = EPI == kQkv ? 4 * kHeadDim + 16 : EPI == kSwiglu ? BN + 16 : 4 * BN + 16;  // bytes
     constexpr int kOutBytes = EPI == kQkv ? BM * kPitch + 4 * BM * 8 : EPI == kSwiglu ? 2 * BM * kPitch : BM * kPitch;
     constexpr int kSmem = NS * kStageBytes > kOutBytes ? NS * kStageBytes : kOutBytes;
