@@ -250,26 +250,34 @@ __global__ __launch_bounds__(256 * HEADS) void attn_prefill_mfma_kernel(const fl
 
     // Direct loads of step i: split sp's tile kt = 4 i + sp; load j of this
     // wave fills 16-byte slot 64 (HEADS j + h) + lane of the K or V tile; rows past
-    // `last` repeat row `last` (masked).
+    // `last` repeat row `last` (masked). The offsets are formed ahead, for all but a
+    // last tile that is not whole: the loads go out together.
     constexpr int kTileLoads = 8 / HEADS;
-    int ld_row[kTileLoads];
-    unsigned ld_col[kTileLoads];
+    unsigned ld_at[kTileLoads];  // bytes from the tile's first row
 #pragma unroll
     for (int j = 0; j < kTileLoads; ++j) {
         const int q = 64 * (HEADS * j + h) + lane, r = q >> 4;
-        ld_row[j] = r;
-        ld_col[j] = 16 * ((q & 15) ^ fb_swz(r));
+        ld_at[j] = r * (kHeadDim * 2) + 16 * ((q & 15) ^ fb_swz(r));
     }
     auto issue = [&](const uint16_t* cache, int step, int v) {
         const int kt = 4 * step + sp;
         const unsigned dst = lds0 + sp * kFbSplitBytes + (2 * v + (step & 1)) * kFbTileBytes + 1024 * h;
-        if (kt < ntiles) {
-            const uint16_t* first = cache + (head_base + size_t(kt) * kFaKeys) * kHeadDim;
-            const int rows_left = last - kt * kFaKeys;  // row `last` of the tile, 31 or more within
+        const int rows_left = last - kt * kFaKeys;  // row `last` of the tile, 31 or more within
+        if (rows_left < 0) return;
+        const uint16_t* first = cache + (head_base + size_t(kt) * kFaKeys) * kHeadDim;
+        auto load = [&](const unsigned* at) {
+#pragma unroll
+            for (int j = 0; j < kTileLoads; j += 4)
+                load4_lds16_opaque<1024 * HEADS>(first, at + j, dst + 1024 * HEADS * j);
+        };
+        if (rows_left >= kFaKeys - 1) {
+            load(ld_at);
+        } else {
+            unsigned at[kTileLoads];
 #pragma unroll
             for (int j = 0; j < kTileLoads; ++j)
-                load_lds16_opaque(first, unsigned(min(ld_row[j], rows_left)) * (kHeadDim * 2) + ld_col[j],
-                                  dst + 1024 * HEADS * j);
+                at[j] = ld_at[j] - max(4 * (HEADS * j + h) + (lane >> 4) - rows_left, 0) * (kHeadDim * 2);
+            load(at);
         }
     };
     issue(keys, 0, 0);
